@@ -423,13 +423,12 @@ int stwo_hip_graph_free(stwo_hip_ctx* ctx, stwo_hip_graph* graph);
  * (11 <= S <= min(k, 15)) and the stages above in strided passes. The context picks S per shape:
  * the largest tile when its grid fills the device four times over, else the fastest candidate,
  * timed once per (device, direction, columns, sizes) and kept in the cache directory
- * (STWO_HIP_KERNEL_CACHE, else ~/.cache/stwo_hip: fft_plans_<arch>_<CUs>.txt). Results never depend
+ * (STWO_HIP_KERNEL_CACHE, else ~/.cache/stwo_hip: fft_plans_<arch>_<CUs>_f64.txt). Results never depend
  * on S. stwo_hip_fft_low_log returns the plan of a shape (tuning it if needed; 0 when the
  * transform has fewer than 11 stages); stwo_hip_set_fft_low_log fixes S for every later transform
  * of the context (clamped to each shape's range; 0 restores planning). A plan may carry the flag
- * 0x100 (S = 15): the low-stage kernel then runs one workgroup per CU, each looping over tiles and
- * loading its next tile while it computes the current one; a transform whose output columns are not
- * all 16-byte aligned runs without it. */
+ * 0x100 (S = 15, forward transforms that fill the device); the low-stage kernel runs the same with
+ * and without it. */
 int stwo_hip_fft_low_log(stwo_hip_ctx* ctx, int inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
                          uint32_t* low_log);
 int stwo_hip_set_fft_low_log(stwo_hip_ctx* ctx, uint32_t low_log);

@@ -17,7 +17,8 @@ using namespace sh;
 
 struct stwo_hip_twiddles {
   uint32_t init_index = 0, log_size = 0;  // the root coset, Coset::new(init_index, log_size)
-  DevBuf tw, itw, tw2, itw2;
+  DevBuf tw, itw, tw2, itw2, twd, itwd;
+  FftTree fft_tree(bool inverse) const { return make_fft_tree(inverse ? itw : tw, inverse ? itw2 : tw2, inverse ? itwd : twd); }
 };
 struct stwo_hip_ctx {
   Ctx* ctx = nullptr;
@@ -89,13 +90,12 @@ void reject_unsatisfied(const stwo_proof& p) {
 // doubled tree whose last 2^(log_n - 1) entries are the domain's line twiddles.
 // `low` is the plan's low-stage tile (Ctx::fft_low_log), taken before the caller's timing scope.
 void run_fft(Ctx& c, bool inverse, const uint32_t* const* ds, uint32_t* const* dd, uint32_t n_cols, uint32_t log_in,
-             uint32_t log_n, const uint32_t* tree2, uint32_t tree_len, uint32_t half_init, uint32_t low) {
+             uint32_t log_n, const FftTree& tree, uint32_t half_init, uint32_t low) {
   if (log_n <= 2) launch_fft_tiny(inverse, ds, dd, n_cols, log_in, log_n, index_to_point(half_init), c.stream);
-  else launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree2, tree_len, c.stream, false, low);
+  else launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, c.stream, false, low);
 }
-uint32_t plan_fft(Ctx& c, bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const uint32_t* tree2,
-                  uint32_t tree_len, uint32_t* const* dst) {
-  return log_n <= 2 ? 0u : Ctx::fft_plan_for(c.fft_low_log(inverse, n_cols, log_in, log_n, tree2, tree_len), dst, n_cols);
+uint32_t plan_fft(Ctx& c, bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree) {
+  return log_n <= 2 ? 0u : c.fft_low_log(inverse, n_cols, log_in, log_n, tree);
 }
 uint32_t canonic_half_init(uint32_t log_n) { return HCoset::half_odds(log_n - 1).initial_index; }
 void check_tree(const stwo_hip_twiddles* t, uint32_t half_init, uint32_t log_n) {
@@ -270,10 +270,10 @@ int stwo_hip_interpolate_columns(stwo_hip_ctx* h, const uint32_t* const* evals, 
     const uint32_t* const* ds = (const uint32_t* const*)c.upload_vec(s);
     uint32_t* const* dd = (uint32_t* const*)c.upload_vec(d);
     {
-      const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, c.itw2.p, c.tree_len(), d.data());
+      const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, c.fft_tree(true));
       KScope ks(c, K_INTERPOLATE, (double)n_cols * 8.0 * (double)(1u << log_size));
       ks.units(fft_butterflies(n_cols, log_size, log_size));
-      run_fft(c, true, ds, dd, n_cols, log_size, log_size, c.itw2.p, c.tree_len(), canonic_half_init(log_size), low);
+      run_fft(c, true, ds, dd, n_cols, log_size, log_size, c.fft_tree(true), canonic_half_init(log_size), low);
     }
     c.end_stream_ordered();
   });
@@ -289,10 +289,10 @@ int stwo_hip_evaluate_polynomials(stwo_hip_ctx* h, const uint32_t* const* coeffs
     const uint32_t* const* ds = (const uint32_t* const*)c.upload_vec(s);
     uint32_t* const* dd = (uint32_t* const*)c.upload_vec(d);
     {
-      const uint32_t low = plan_fft(c, false, n_cols, log_size, log_n, c.tw2.p, c.tree_len(), d.data());
+      const uint32_t low = plan_fft(c, false, n_cols, log_size, log_n, c.fft_tree(false));
       KScope ks(c, K_EVALUATE, (double)n_cols * (4.0 * (double)(1u << log_size) + 4.0 * (double)(1u << log_n)));
       ks.units(fft_butterflies(n_cols, log_n, log_size));
-      run_fft(c, false, ds, dd, n_cols, log_size, log_n, c.tw2.p, c.tree_len(), canonic_half_init(log_n), low);
+      run_fft(c, false, ds, dd, n_cols, log_size, log_n, c.fft_tree(false), canonic_half_init(log_n), low);
     }
     c.end_stream_ordered();
   });
@@ -1136,7 +1136,7 @@ int stwo_hip_twiddles_create(stwo_hip_ctx* h, uint32_t coset_initial_index, uint
     auto t = std::make_unique<stwo_hip_twiddles>();
     t->init_index = coset_initial_index & 0x7fffffffu;
     t->log_size = coset_log_size;
-    build_twiddle_tree(c, t->init_index, coset_log_size, t->tw, t->itw, t->tw2, t->itw2);
+    build_twiddle_tree(c, t->init_index, coset_log_size, t->tw, t->itw, t->tw2, t->itw2, t->twd, t->itwd);
     h->trees.insert(t.get());
     *out = t.release();
   });
@@ -1166,11 +1166,11 @@ int stwo_hip_interpolate_on_domain(stwo_hip_ctx* h, const stwo_hip_twiddles* t, 
     std::vector<const uint32_t*> s(evals, evals + n_cols);
     std::vector<uint32_t*> d(coeffs, coeffs + n_cols);
     {
-      const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, t->itw2.p, 1u << t->log_size, d.data());
+      const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, t->fft_tree(true));
       KScope ks(c, K_INTERPOLATE, (double)n_cols * 8.0 * (double)(1u << log_size));
       ks.units(fft_butterflies(n_cols, log_size, log_size));
       run_fft(c, true, (const uint32_t* const*)c.upload_vec(s), (uint32_t* const*)c.upload_vec(d), n_cols, log_size,
-              log_size, t->itw2.p, 1u << t->log_size, half_coset_initial_index, low);
+              log_size, t->fft_tree(true), half_coset_initial_index, low);
     }
     c.end_stream_ordered();
   });
@@ -1186,11 +1186,11 @@ int stwo_hip_evaluate_on_domain(stwo_hip_ctx* h, const stwo_hip_twiddles* t, uin
     std::vector<const uint32_t*> s(coeffs, coeffs + n_cols);
     std::vector<uint32_t*> d(evals, evals + n_cols);
     {
-      const uint32_t low = plan_fft(c, false, n_cols, log_coeffs, log_size, t->tw2.p, 1u << t->log_size, d.data());
+      const uint32_t low = plan_fft(c, false, n_cols, log_coeffs, log_size, t->fft_tree(false));
       KScope ks(c, K_EVALUATE, (double)n_cols * (4.0 * (double)(1u << log_coeffs) + 4.0 * (double)(1u << log_size)));
       ks.units(fft_butterflies(n_cols, log_size, log_coeffs));
       run_fft(c, false, (const uint32_t* const*)c.upload_vec(s), (uint32_t* const*)c.upload_vec(d), n_cols, log_coeffs,
-              log_size, t->tw2.p, 1u << t->log_size, half_coset_initial_index, low);
+              log_size, t->fft_tree(false), half_coset_initial_index, low);
     }
     c.end_stream_ordered();
   });
@@ -1438,8 +1438,8 @@ int stwo_hip_fft_low_log(stwo_hip_ctx* h, int inverse, uint32_t n_cols, uint32_t
     *low_log = 0;
     if (log_n <= 2 || n_cols == 0) return;
     c.ensure_twiddles(log_n);
-    *low_log = inverse ? c.fft_low_log(true, n_cols, log_in, log_n, c.itw2.p, c.tree_len())
-                       : c.fft_low_log(false, n_cols, log_in, log_n, c.tw2.p, c.tree_len());
+    *low_log = inverse ? c.fft_low_log(true, n_cols, log_in, log_n, c.fft_tree(true))
+                       : c.fft_low_log(false, n_cols, log_in, log_n, c.fft_tree(false));
     c.sync();
   });
 }

@@ -13,10 +13,12 @@ namespace sh {
 // first half of the coset doubled j times, bit-reversed, at [2^L - 2^(L-j), 2^L - 2^(L-j-1)); the
 // last entry is the pad 1. Point k of the coset doubled j times has index
 // (init + k 2^(31-L)) 2^j, and the point of an index is the sum of the generator's powers 2^b
-// over its set bits. Inverses by Fermat; the doubled trees hold 2t. A zero x-coordinate (which
+// over its set bits. Inverses by Fermat; the doubled trees hold 2t, and twd and
+// itwd the last n_d entries as doubles. A zero x-coordinate (which
 // has no inverse) raises *zero_flag.
 __global__ void __launch_bounds__(256) twiddle_tree_kernel(uint32_t init, uint32_t L, GenPowers g, uint32_t* tw,
                                                            uint32_t* itw, uint32_t* tw2, uint32_t* itw2,
+                                                           double* twd, double* itwd, uint32_t n_d,
                                                            uint32_t* zero_flag) {
   const uint32_t len = 1u << L;
   for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < len; e += gridDim.x * blockDim.x) {
@@ -38,18 +40,22 @@ __global__ void __launch_bounds__(256) twiddle_tree_kernel(uint32_t init, uint32
     itw[e] = xi;
     tw2[e] = 2 * x;
     itw2[e] = 2 * xi;
+    if (e >= len - n_d) {
+      twd[e - (len - n_d)] = (double)x;
+      itwd[e - (len - n_d)] = (double)xi;
+    }
   }
 }
 
 void launch_twiddle_tree(uint32_t init_index, uint32_t log_size, uint32_t* tw, uint32_t* itw, uint32_t* tw2,
-                         uint32_t* itw2, uint32_t* zero_flag, hipStream_t stream) {
+                         uint32_t* itw2, double* twd, double* itwd, uint32_t* zero_flag, hipStream_t stream) {
   GenPowers g;
   cpm31 c = circle_gen();
   for (int b = 0; b < 31; ++b) { g.p[b] = c; c = cp_double(c); }
   const size_t len = (size_t)1 << log_size;
   const uint32_t blocks = (uint32_t)((len + 255) / 256 < 8192 ? (len + 255) / 256 : 8192);
   hipLaunchKernelGGL(twiddle_tree_kernel, dim3(blocks), dim3(256), 0, stream, init_index & 0x7fffffffu, log_size, g, tw,
-                     itw, tw2, itw2, zero_flag);
+                     itw, tw2, itw2, twd, itwd, (uint32_t)fft_tree_doubles(len), zero_flag);
 }
 
 // In-place bit reversal: the lane of the smaller index of each swapped pair moves both words.

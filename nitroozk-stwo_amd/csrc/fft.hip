@@ -8,9 +8,10 @@
 // 2^b-times larger domain skips the top b stages: on zero-padded input they only copy, so the
 // first pass reads the coefficient column with the index masked to 2^k.
 //
-// MI355X mapping: one workgroup owns a tile of 2^S * 2^c words in LDS and runs S consecutive
-// stages on it. The first (lowest) stages use contiguous tiles (c = 0); higher stages use
-// strided tiles made of 2^c adjacent sub-columns so that global loads stay coalesced.
+// MI355X mapping, by transform size k (stages that run):
+//   k >= 11   the low 11..15 stages in one pass over a tile in LDS, on doubles (fft_low_kernel);
+//             the stages above in passes of at most 6 on register-resident words (fft_pass_reg_kernel)
+//   k < 11    one or two passes on a tile in LDS (fft_pass_kernel)
 #include <stdexcept>
 #include "butterfly.h"
 #include "field.h"
@@ -161,10 +162,14 @@ constexpr uint32_t PASS_REG_MAX = 6;  // stages per register pass (2^S values pe
 // ---- low stages of a 2^S-element block in one pass (11 <= S <= 15) ---------------------------
 // A workgroup of 2^(S-5) threads owns one block (tile) of 2^S consecutive elements of one column
 // and runs stages [0, S) on it as three rounds (bits 0-4, 5-9, 10..S-1); in a round each thread
-// holds 32 elements in registers and runs up to 5 stages on them. The first round reads its
-// elements straight from global memory and the last round writes its results straight back; only
-// the hand-overs between rounds go through LDS, where word e lives at e + e/32 so that every
-// round's accesses are free of bank conflicts.
+// holds 32 elements in registers, as doubles (butterfly.h), and runs up to 5 stages on them. The
+// first round reads its elements straight from global memory and the last round writes its results
+// straight back; the hand-overs between rounds go through LDS as 32-bit words (pack_f64), where word
+// e lives at e + e/32 so that every round's accesses are free of bank conflicts.
+//
+// In the rounds at bits 0 and 5 a wave owns the same 2048 consecutive elements, so the hand-over
+// between them stays inside the wave: no workgroup barrier, only the one between the rounds at bits
+// 5 and 10.
 //
 // Workgroups go to the 8 XCDs in turn (workgroup n to XCD n mod 8). Renumbering them so that each
 // XCD takes a contiguous range of tiles keeps the tiles of one column on one XCD and its L2: when
@@ -172,395 +177,368 @@ constexpr uint32_t PASS_REG_MAX = 6;  // stages per register pass (2^S values pe
 // the first read reaches HBM.
 __device__ __forceinline__ uint32_t lds_pad(uint32_t e) { return e + (e >> 5); }
 
-// Threads per workgroup and element registers per thread for a tile of 2^S elements.
-template <int S> struct LowShape {
-  static constexpr int X = 0;                       // 2^X groups of 32 elements per thread
-  static constexpr uint32_t T = 1u << (S - 5 - X);
-  static constexpr uint32_t V = 32u << X;
-};
+// Threads per workgroup for a tile of 2^S elements, 32 per thread.
+template <int S> constexpr uint32_t LOW_T = 1u << (S - 5);
 
-// Element (within the tile) held in register slot g * 2^R + q by thread t in the round at bit A.
-template <int S, int A, int R>
-__device__ __forceinline__ uint32_t round_elem(uint32_t t, uint32_t g, uint32_t q) {
-  constexpr uint32_t T = LowShape<S>::T;
-  const uint32_t rho = t + g * T;
-  return ((rho >> A) << (A + R)) | (rho & ((1u << A) - 1)) | (q << A);
+// In the round at bit A a lane's register slot g 2^R + q holds the element
+// lane_elem + g LOW_T + (q << A) (g > 0 in rounds at bit 10 of fewer than 5 stages only). All slots of a
+// lane sit at fixed distances, in the tile and in LDS, so that an access is one base address and an
+// immediate offset.
+template <int A> __device__ __forceinline__ uint32_t lane_elem(uint32_t t) {
+  return A == 0 ? t << 5 : A == 5 ? ((t >> 5) << 10) | (t & 31) : t;
+}
+template <int S, int A> __device__ __forceinline__ constexpr uint32_t slot_lds(uint32_t g, uint32_t q) {
+  return g * (LOW_T<S> + (LOW_T<S> >> 5)) + q * (A == 0 ? 1u : (1u << A) + (1u << A >> 5));
 }
 
-// With one group per lane and A >= 5, slot q's element is the lane's first element plus q 2^A
-// (no carries into the lane's bits), and its padded LDS word is the first one's plus
-// q (2^A + 2^(A-5)): one base address per lane and immediate offsets, instead of three
-// instructions of index arithmetic per slot.
-template <int S, int A, int R>
-constexpr bool LDS_AFFINE = A >= 5 && ((1u << (5 - R)) << LowShape<S>::X) == 1;
-template <int S, int A, int R>
-__device__ __forceinline__ void round_from_lds(uint32_t* v, const uint32_t* lds) {
-  constexpr uint32_t G = (1u << (5 - R)) << LowShape<S>::X, Q = 1u << R;
-  if constexpr (LDS_AFFINE<S, A, R>) {
-    const uint32_t* b = lds + lds_pad(round_elem<S, A, R>(threadIdx.x, 0, 0));
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) v[q] = b[q * ((1u << A) + (1u << (A - 5)))];
-    return;
-  }
-#pragma unroll
-  for (uint32_t g = 0; g < G; ++g)
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) v[g * Q + q] = lds[lds_pad(round_elem<S, A, R>(threadIdx.x, g, q))];
-}
-template <int S, int A, int R>
-__device__ __forceinline__ void round_to_lds(const uint32_t* v, uint32_t* lds) {
-  constexpr uint32_t G = (1u << (5 - R)) << LowShape<S>::X, Q = 1u << R;
-  if constexpr (LDS_AFFINE<S, A, R>) {
-    uint32_t* b = lds + lds_pad(round_elem<S, A, R>(threadIdx.x, 0, 0));
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) b[q * ((1u << A) + (1u << (A - 5)))] = v[q];
-    return;
-  }
-#pragma unroll
-  for (uint32_t g = 0; g < G; ++g)
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) lds[lds_pad(round_elem<S, A, R>(threadIdx.x, g, q))] = v[g * Q + q];
-}
-// Global elements gbase | e (index masked with in_mask) of the round's slots. At A = 0 a thread's
-// 32 elements are consecutive: 16-byte loads when the column allows them.
-// Rounds whose lanes own the 2^A low bits of the tile index (A = 10 with 1024 lanes): element q
-// of lane t is the tile's word t + q 2^A, so a buffer access takes the lane offset in a vector
-// register and the element offset in a scalar one, with no vector address arithmetic.
-template <int S, int A> constexpr bool LANE_LOW_BITS = LowShape<S>::X == 0 && LowShape<S>::T == (1u << A);
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t column_rsrc(const void* p, uint32_t words) {
-  // raw buffer over the column (stride 0, 32-bit data format); accesses past `words` read 0
-  const uint32_t bytes = words >= (1u << 30) ? 0xffffffffu : words * 4u;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+// Orders a wave's LDS writes before its later LDS reads (other lanes' words): the LDS serves a wave's
+// accesses in order, so only the compiler has to be held back.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 template <int S, int A, int R>
-__device__ __forceinline__ void round_from_global(uint32_t* v, const GLOBAL_AS uint32_t* __restrict__ in, uint32_t gbase,
-                                                  uint32_t in_mask, bool vec) {
-  constexpr uint32_t G = (1u << (5 - R)) << LowShape<S>::X, Q = 1u << R;
-  if constexpr (LANE_LOW_BITS<S, A>) {
-    // (gbase | t | q 2^A) & in_mask with in_mask >= 2^S - 1: the tile's base is gbase & in_mask
-    const __amdgpu_buffer_rsrc_t rs = column_rsrc((const void*)in, in_mask + 1);
-    const uint32_t base = __builtin_amdgcn_readfirstlane(gbase & in_mask);
+__device__ __forceinline__ void round_from_lds(double* w, const uint32_t* lds, uint32_t t) {
+  const uint32_t* b = lds + lds_pad(lane_elem<A>(t));
 #pragma unroll
-    for (uint32_t q = 0; q < Q; ++q)
-      v[q] = __builtin_amdgcn_raw_buffer_load_b32(rs, threadIdx.x * 4u, (base + (q << A)) * 4u, 0);
-    return;
+  for (uint32_t g = 0; g < (1u << (5 - R)); ++g)
+#pragma unroll
+    for (uint32_t q = 0; q < (1u << R); ++q) w[(g << R) + q] = (double)b[slot_lds<S, A>(g, q)];
+}
+template <int S, int A, int R>
+__device__ __forceinline__ void round_to_lds(const double* w, uint32_t* lds, uint32_t t) {
+  uint32_t* b = lds + lds_pad(lane_elem<A>(t));
+#pragma unroll
+  for (uint32_t g = 0; g < (1u << (5 - R)); ++g)
+#pragma unroll
+    for (uint32_t q = 0; q < (1u << R); ++q) b[slot_lds<S, A>(g, q)] = pack_f64(w[(g << R) + q]);
+}
+// The round at bit 10 reads and writes its elements in rows of 2^(S-5) lanes: a buffer access takes
+// the lane offset in a vector register and the slot's in a scalar one, with no vector address
+// arithmetic.
+// A raw buffer over `words` words at p: past them, loads read 0 and stores are dropped. Address and
+// size are the same for the whole wave: said so, they stay in scalar registers.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const GLOBAL_AS uint32_t* p, uint32_t words) {
+  const uint64_t a = (uint64_t)p;
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(hi << 32 | lo), (short)0,
+                                           (int)__builtin_amdgcn_readfirstlane(words * 4u), 0x00020000);
+}
+template <int S>
+__device__ __forceinline__ void load_round10(uint32_t* v, const GLOBAL_AS uint32_t* in, uint32_t t) {
+  constexpr int R = S - 10;
+  const __amdgpu_buffer_rsrc_t rs = tile_rsrc(in, 1u << S);
+#pragma unroll
+  for (uint32_t g = 0; g < (1u << (5 - R)); ++g)
+#pragma unroll
+    for (uint32_t q = 0; q < (1u << R); ++q)
+      v[(g << R) + q] = __builtin_amdgcn_raw_buffer_load_b32(rs, t * 4u, (g * LOW_T<S> + (q << 10)) * 4u, 0);
+}
+template <int S>
+__device__ __forceinline__ void store_round10(const uint32_t* v, GLOBAL_AS uint32_t* out, uint32_t out_words, uint32_t t) {
+  constexpr int R = S - 10;
+  const __amdgpu_buffer_rsrc_t rs = tile_rsrc(out, out_words);
+#pragma unroll
+  for (uint32_t g = 0; g < (1u << (5 - R)); ++g)
+#pragma unroll
+    for (uint32_t q = 0; q < (1u << R); ++q)
+      __builtin_amdgcn_raw_buffer_store_b32(v[(g << R) + q], rs, t * 4u, (g * LOW_T<S> + (q << 10)) * 4u, 0);
+}
+// 16-byte accesses to columns that may be aligned to 4 bytes only: the device takes them at any word.
+typedef u32x4 u32x4_w __attribute__((aligned(4)));
+// The round at bit 0 reads 32 consecutive elements per lane.
+__device__ __forceinline__ void load_round0(uint32_t* v, const GLOBAL_AS uint32_t* in, uint32_t t) {
+  const GLOBAL_AS u32x4_w* b = reinterpret_cast<const GLOBAL_AS u32x4_w*>(in + (t << 5));
+#pragma unroll
+  for (uint32_t m = 0; m < 8; ++m) {
+    const u32x4 x = b[m];
+    v[4 * m] = x.x; v[4 * m + 1] = x.y; v[4 * m + 2] = x.z; v[4 * m + 3] = x.w;
   }
-  if (A == 0 && R == 5 && vec) {
+}
+__device__ __forceinline__ void to_f64(double* w, const uint32_t* v) {
+#pragma unroll
+  for (uint32_t i = 0; i < 32; ++i) w[i] = (double)v[i];
+}
+// A last round's results, canonical; rot != 0 multiplies them by 2^rot, which rotates the 31-bit word
+// (2^-log_n is 2^(31 - log_n)).
+__device__ __forceinline__ void canon_words(uint32_t* v, const double* w, uint32_t rot) {
+#pragma unroll
+  for (uint32_t i = 0; i < 32; ++i) v[i] = canon_f64(w[i]);
+  if (rot) {
+#pragma unroll
+    for (uint32_t i = 0; i < 32; ++i) v[i] = m31_rotl(v[i], rot);
+  }
+}
+// The results of a last round at bit 0, canonical. A lane holds 32 consecutive words, and storing them
+// from there would put 64 pieces of 16 bytes into 64 lines with every instruction. They cross the
+// wave's own part of LDS instead (its 2048 words; 16-byte unit c of lane l at unit 8 l + (c ^ (l & 7)),
+// free of bank conflicts both ways), so that an instruction stores 1 KB in a row: memory traffic alone,
+// 497 MB, 92 us against 123. Streaming stores (aux 2): nothing of the tile is read again by this
+// kernel, and the traffic alone takes 73 us.
+__device__ __forceinline__ u32x4* wave_units(uint32_t* lds, uint32_t t) {
+  return reinterpret_cast<u32x4*>(lds + lds_pad((t & ~63u) << 5));
+}
+__device__ __forceinline__ void round0_stage_out(const double* w, uint32_t* lds, uint32_t t) {
+  uint32_t v[32];
+  canon_words(v, w, 0);
+  const uint32_t l = t & 63;
+  u32x4* own = wave_units(lds, t);
+#pragma unroll
+  for (uint32_t c = 0; c < 8; ++c) own[8 * l + (c ^ (l & 7))] = u32x4{v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
+  wave_lds_fence();
+}
+__device__ __forceinline__ void store_round0(uint32_t* lds, GLOBAL_AS uint32_t* out, uint32_t out_words, uint32_t t) {
+  const uint32_t l = t & 63, r = l >> 3;  // unit (l & 7) of lane 8 k + r
+  const u32x4* own = wave_units(lds, t);
+  const __amdgpu_buffer_rsrc_t rs = tile_rsrc(out, out_words);
+  const uint32_t base = __builtin_amdgcn_readfirstlane((t & ~63u) << 5);
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k)
+    __builtin_amdgcn_raw_buffer_store_b128(own[8 * (8 * k + r) + ((l & 7) ^ r)], rs, l * 16u, (base + 256 * k) * 4u, 2);
+}
+
+// Twiddles. Stage s >= 1 of the pair whose lower element is idx reads entry idx >> (s + 1) of the
+// 2^(log_n - s) entries that end the tree (tree.end - 2^(log_n - s)).
+//
+// The round at bit 10: the lanes own bits below the round, so the workgroup shares its twiddles, and
+// they come as doubles through the scalar cache.
+template <bool INV, int S, int R>
+__device__ __forceinline__ void round10_butterflies(double* w, uint32_t gbase, const double* __restrict__ td_end,
+                                                    uint32_t log_n, double M) {
+  constexpr uint32_t G = 1u << (5 - R), Q = 1u << R;
+#pragma unroll
+  for (int kk = 0; kk < R; ++kk) {
+    const int k = INV ? kk : R - 1 - kk;
+    const uint32_t s = 10 + k;
 #pragma unroll
     for (uint32_t g = 0; g < G; ++g) {
-      const uint32_t e0 = 32 * (threadIdx.x + g * LowShape<S>::T);
-#pragma unroll
-      for (uint32_t m = 0; m < 8; ++m) {
-        const u32x4 w = *reinterpret_cast<const GLOBAL_AS u32x4*>(in + ((gbase | (e0 + 4 * m)) & in_mask));
-        v[32 * g + 4 * m] = w.x; v[32 * g + 4 * m + 1] = w.y; v[32 * g + 4 * m + 2] = w.z; v[32 * g + 4 * m + 3] = w.w;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (uint32_t g = 0; g < G; ++g)
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) v[g * Q + q] = in[(gbase | round_elem<S, A, R>(threadIdx.x, g, q)) & in_mask];
-}
-// ALWAYS_VEC: the caller guarantees 16-byte aligned columns, and the round at bit 0 stores with
-// 16-byte writes on one code path.
-template <int S, int A, int R, bool ALWAYS_VEC = false>
-__device__ __forceinline__ void round_to_global(uint32_t* v, GLOBAL_AS uint32_t* __restrict__ out, uint32_t gbase,
-                                                uint32_t scale, bool vec, uint32_t out_words) {
-  constexpr uint32_t G = (1u << (5 - R)) << LowShape<S>::X, Q = 1u << R;
-  if (scale) {
-#pragma unroll
-    for (uint32_t i = 0; i < LowShape<S>::V; ++i) v[i] = mul_tw(v[i], scale);
-  }
-  if constexpr (LANE_LOW_BITS<S, A>) {
-    const __amdgpu_buffer_rsrc_t rs = column_rsrc((const void*)out, out_words);
-    const uint32_t base = __builtin_amdgcn_readfirstlane(gbase);
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q)
-      __builtin_amdgcn_raw_buffer_store_b32(v[q], rs, threadIdx.x * 4u, (base + (q << A)) * 4u, 0);
-    return;
-  }
-  if (A == 0 && R == 5 && (ALWAYS_VEC || vec)) {
-#pragma unroll
-    for (uint32_t g = 0; g < G; ++g) {
-      const uint32_t e0 = 32 * (threadIdx.x + g * LowShape<S>::T);
-#pragma unroll
-      for (uint32_t m = 0; m < 8; ++m)
-        *reinterpret_cast<GLOBAL_AS u32x4*>(out + (gbase | (e0 + 4 * m))) =
-            u32x4{v[32 * g + 4 * m], v[32 * g + 4 * m + 1], v[32 * g + 4 * m + 2], v[32 * g + 4 * m + 3]};
-    }
-    return;
-  }
-#pragma unroll
-  for (uint32_t g = 0; g < G; ++g)
-#pragma unroll
-    for (uint32_t q = 0; q < Q; ++q) out[gbase | round_elem<S, A, R>(threadIdx.x, g, q)] = v[g * Q + q];
-}
-
-// The R stages of the round at bit A on the registers (2^(R-1) * R butterflies per group, one
-// twiddle per distinct butterfly block).
-template <bool INV, int S, int A, int R>
-__device__ __forceinline__ void round_butterflies(uint32_t* v, uint32_t gbase, const uint32_t* __restrict__ tree,
-                                                  uint32_t tree_len, uint32_t log_n) {
-  constexpr uint32_t T = LowShape<S>::T, G = (1u << (5 - R)) << LowShape<S>::X, Q = 1u << R;
-  const uint32_t t = threadIdx.x;
-#pragma unroll
-  for (uint32_t g = 0; g < G; ++g) {
-    const uint32_t rho = t + g * T;
-    const uint32_t idx_base = gbase | ((rho >> A) << (A + R)) | (rho & ((1u << A) - 1));
-#pragma unroll
-    for (int kk = 0; kk < R; ++kk) {
-      const int k = INV ? kk : R - 1 - kk;
-      const uint32_t s = A + k;
-      if (A == 0 && k == 0) {
-        // stage 0: pair h = (idx_base >> 1) | u, whose quarter u & 3 is known here, so the negated
-        // circle twiddles become swapped additions
-        // pair h = (idx_base >> 1) + u (idx_base's low 5 bits are zero): its [x, y] twiddle pair is
-        // at 2 (h >> 2) = 2 (idx_base >> 3) + 2 (u >> 2)
-        const uint32_t* lb = tree + tree_len - (1u << (log_n - 1)) + 2 * (idx_base >> 3);
-#pragma unroll
-        for (uint32_t u = 0; u < (Q >> 1); u += 4) {
-          const uint32_t x = lb[2 * (u >> 2)], y = lb[2 * (u >> 2) + 1];
-          bfly<INV, false>(v[g * Q + 2 * u], v[g * Q + 2 * u + 1], y);
-          bfly<INV, true>(v[g * Q + 2 * u + 2], v[g * Q + 2 * u + 3], y);
-          bfly<INV, true>(v[g * Q + 2 * u + 4], v[g * Q + 2 * u + 5], x);
-          bfly<INV, false>(v[g * Q + 2 * u + 6], v[g * Q + 2 * u + 7], x);
-        }
-        continue;
-      }
-      // stage s >= 1: the twiddle of block u is tree[len - 2^(log_n - s) + (idx_base >> (s + 1)) + u]
-      // (idx_base is zero on the round's bits, so u adds without carries): one base per stage
-      // (when the lanes' bits all lie below bit A, the base is the same for the whole workgroup and
-      // the twiddles come through the scalar cache)
-      constexpr bool UNIFORM_TW = T * G <= (1u << A);
-      // The round at bit 5 with one group per lane: the lanes' bits above the round are t >> 5, two
-      // values in a wave (its halves), so both halves' twiddles load through the scalar cache (the
-      // upper half's 2^(R-1-k) entries further on) and each lane selects its own. No vector load
-      // waits here on older loads and stores still in flight.
-      constexpr bool HALF_TW = !UNIFORM_TW && A == 5 && G == 1;
-      const uint32_t toff = (UNIFORM_TW || HALF_TW) ? __builtin_amdgcn_readfirstlane(idx_base >> (s + 1))
-                                                    : idx_base >> (s + 1);
-      const uint32_t* tb = tree + tree_len - (1u << (log_n - s)) + toff;
-      const bool upper = (threadIdx.x & 32) != 0;
+      // group g's lanes: bits 0..9 and, for tiles below 2^15, none above the round (T G = 2^10)
+      const double* tb = td_end - (1u << (log_n - s)) + __builtin_amdgcn_readfirstlane(gbase >> (s + 1));
 #pragma unroll
       for (uint32_t u = 0; u < (Q >> (k + 1)); ++u) {
-        uint32_t tw;
-        if constexpr (HALF_TW) {
-          // both values made wave-uniform, so that the select is not folded into one per-lane load
-          const uint32_t lo = __builtin_amdgcn_readfirstlane(tb[u]);
-          const uint32_t hi = __builtin_amdgcn_readfirstlane(tb[u + (1u << (R - 1 - k))]);
-          tw = upper ? hi : lo;
-        } else {
-          tw = tb[u];
-        }
+        const double tw = tb[u];
 #pragma unroll
         for (uint32_t l = 0; l < (1u << k); ++l) {
           const uint32_t q = (u << (k + 1)) | l;
-          bfly<INV>(v[g * Q + q], v[g * Q + (q | (1u << k))], tw);
+          bfly_f64<INV>(w[g * Q + q], w[g * Q + (q | (1u << k))], tw, M);
         }
       }
     }
   }
 }
 
-template <bool INV, int S>
-__global__ void __launch_bounds__(LowShape<S>::T) fft_low_kernel(const uint32_t* const* __restrict__ src,
-                                                                 uint32_t* const* __restrict__ dst, uint32_t log_n,
-                                                                 uint32_t in_mask, const uint32_t* __restrict__ tree,
-                                                                 uint32_t tree_len, uint32_t scale, uint32_t prio) {
-  if (prio) CRITICAL_PATH_WAVE();
-  constexpr uint32_t N = 1u << S;
-  // rounds in execution order: the inverse runs bits 0-4, 5-9, 10..S-1; the forward the reverse
-  constexpr int A1 = INV ? 0 : 10, R1 = INV ? 5 : S - 10;
-  constexpr int A3 = INV ? 10 : 0, R3 = INV ? S - 10 : 5;
-  __shared__ uint32_t lds[N + (N >> 5)];
-  const uint32_t n_wg = gridDim.x, hw = blockIdx.x;
-  const uint32_t tile = (n_wg & 7) == 0 ? (hw & 7) * (n_wg >> 3) + (hw >> 3) : hw;
-  const uint32_t blk_log = log_n - S;
-  const uint32_t col = tile >> blk_log, gbase = (tile & ((1u << blk_log) - 1)) << S;
-  const GLOBAL_AS uint32_t* __restrict__ in = gmem(src[col]);
-  GLOBAL_AS uint32_t* __restrict__ out = gmem(dst[col]);
-  uint32_t v[LowShape<S>::V];
-  round_from_global<S, A1, R1>(v, in, gbase, in_mask, (reinterpret_cast<uintptr_t>(in) & 15) == 0);
-  round_butterflies<INV, S, A1, R1>(v, gbase, tree, tree_len, log_n);
-  round_to_lds<S, A1, R1>(v, lds);
-  __syncthreads();
-  round_from_lds<S, 5, 5>(v, lds);
-  round_butterflies<INV, S, 5, 5>(v, gbase, tree, tree_len, log_n);
-  round_to_lds<S, 5, 5>(v, lds);
-  __syncthreads();
-  round_from_lds<S, A3, R3>(v, lds);
-  round_butterflies<INV, S, A3, R3>(v, gbase, tree, tree_len, log_n);
-  round_to_global<S, A3, R3>(v, out, gbase, scale, (reinterpret_cast<uintptr_t>(out) & 15) == 0, 1u << log_n);
+// The round at bit 5: 31 twiddles for each 2^10 consecutive elements, which are half a wave, kept in
+// LDS: those of stage 5 + k of block b at [33 b + 2^(4-k), 33 b + 2^(5-k)). Each wave fills the entries
+// of its own two blocks, one per lane, so no barrier is needed either.
+constexpr uint32_t TW5_STRIDE = 33;
+__device__ __forceinline__ double load_tw5(uint32_t gbase, const double* __restrict__ td_end, uint32_t log_n,
+                                                uint32_t t) {
+  const uint32_t b = t >> 5, j = t & 31;
+  const uint32_t lg = j ? 31u - __builtin_clz(j) : 0u, s = 9 - lg;  // stage 5 + k with k = 4 - lg
+  return gmem(td_end)[(int)((gbase >> (s + 1)) + (b << lg) + (j ? j - (1u << lg) : 0u)) - (1 << (log_n - s))];
+}
+__device__ __forceinline__ void store_tw5(double* tw5, double x, uint32_t t) {
+  tw5[TW5_STRIDE * (t >> 5) + (t & 31)] = x;  // entry 0 of a block is not read
+}
+template <bool INV>
+__device__ __forceinline__ void round5_butterflies(double* w, const double* tw5, double M, uint32_t t) {
+  const double* tb = tw5 + TW5_STRIDE * (t >> 5);
+#pragma unroll
+  for (int kk = 0; kk < 5; ++kk) {
+    const int k = INV ? kk : 4 - kk;
+#pragma unroll
+    for (uint32_t u = 0; u < (16u >> k); ++u) {
+      const double tw = tb[(16u >> k) + u];
+#pragma unroll
+      for (uint32_t l = 0; l < (1u << k); ++l) {
+        const uint32_t q = (u << (k + 1)) | l;
+        bfly_f64<INV>(w[q], w[q | (1u << k)], tw, M);
+      }
+    }
+  }
 }
 
-// The per-lane twiddles of the round at bit 0 (R = 5, one group per lane), loaded ahead of the
-// butterflies: stage 0's circle pairs (x, y) for its four quarters, then the line twiddles of
-// stages 1..4 (8 + 4 + 2 + 1, stage k from 16 - 2^(5-k)).
+// The round at bit 0: a lane's own twiddles, as words (converted where they are used). Stage 0's pairs
+// [x, y] (each for four circle pairs, whose twiddles are y, -y, -x, x: the negated ones become swapped
+// additions), then those of stages 1..4 (8 + 4 + 2 + 1, stage k from 16 - 2^(5-k)).
 struct Round0Tw {
-  uint32_t cx[4], cy[4], t[15];
+  u32x4 c[2];
+  u32x4 t1[2], t2;
+  u32x2 t3;
+  uint32_t t4;
 };
-template <int S>
-__device__ __forceinline__ void load_round0_tw(Round0Tw& tw, uint32_t gbase, const uint32_t* __restrict__ tree,
-                                               uint32_t tree_len, uint32_t log_n) {
-  static_assert(LowShape<S>::X == 0, "one group per lane");
-  const uint32_t idx_base = gbase | (threadIdx.x << 5);
-  const uint32_t* lb = tree + tree_len - (1u << (log_n - 1)) + 2 * (idx_base >> 3);
-#pragma unroll
-  for (uint32_t j = 0; j < 4; ++j) {
-    tw.cx[j] = lb[2 * j];
-    tw.cy[j] = lb[2 * j + 1];
-  }
-#pragma unroll
-  for (uint32_t k = 1; k < 5; ++k) {
-    const uint32_t* tb = tree + tree_len - (1u << (log_n - k)) + (idx_base >> (k + 1));
-#pragma unroll
-    for (uint32_t u = 0; u < (16u >> k); ++u) tw.t[16 - (32u >> k) + u] = tb[u];
-  }
+__device__ __forceinline__ void load_round0_tw(Round0Tw& tw, uint32_t gbase, const uint32_t* __restrict__ t_end,
+                                               uint32_t log_n, uint32_t t) {
+  // the lane's first element is a multiple of 32, so every group of entries is aligned to its size
+  const uint32_t idx = gbase | (t << 5);
+  const auto at = [&](uint32_t s) { return gmem(t_end) - (1u << (log_n - s)) + (idx >> (s + 1)); };
+  const GLOBAL_AS uint32_t* c = gmem(t_end) - (1u << (log_n - 1)) + 2 * (idx >> 3);
+  tw.c[0] = *reinterpret_cast<const GLOBAL_AS u32x4*>(c);
+  tw.c[1] = *reinterpret_cast<const GLOBAL_AS u32x4*>(c + 4);
+  tw.t1[0] = *reinterpret_cast<const GLOBAL_AS u32x4*>(at(1));
+  tw.t1[1] = *reinterpret_cast<const GLOBAL_AS u32x4*>(at(1) + 4);
+  tw.t2 = *reinterpret_cast<const GLOBAL_AS u32x4*>(at(2));
+  tw.t3 = *reinterpret_cast<const GLOBAL_AS u32x2*>(at(3));
+  tw.t4 = *at(4);
 }
-// round_butterflies<INV, S, 0, 5> with the twiddles of load_round0_tw.
 template <bool INV>
-__device__ __forceinline__ void round0_butterflies_pre(uint32_t* v, const Round0Tw& tw) {
+__device__ __forceinline__ void round0_butterflies(double* w, const Round0Tw& tw, double M) {
 #pragma unroll
   for (int kk = 0; kk < 5; ++kk) {
     const int k = INV ? kk : 4 - kk;
     if (k == 0) {
 #pragma unroll
-      for (uint32_t u = 0; u < 16; u += 4) {
-        const uint32_t x = tw.cx[u >> 2], y = tw.cy[u >> 2];
-        bfly<INV, false>(v[2 * u], v[2 * u + 1], y);
-        bfly<INV, true>(v[2 * u + 2], v[2 * u + 3], y);
-        bfly<INV, true>(v[2 * u + 4], v[2 * u + 5], x);
-        bfly<INV, false>(v[2 * u + 6], v[2 * u + 7], x);
+      for (uint32_t u = 0; u < 4; ++u) {
+        const double x = (double)tw.c[u >> 1][2 * (u & 1)], y = (double)tw.c[u >> 1][2 * (u & 1) + 1];
+        bfly_f64<INV, false>(w[8 * u], w[8 * u + 1], y, M);
+        bfly_f64<INV, true>(w[8 * u + 2], w[8 * u + 3], y, M);
+        bfly_f64<INV, true>(w[8 * u + 4], w[8 * u + 5], x, M);
+        bfly_f64<INV, false>(w[8 * u + 6], w[8 * u + 7], x, M);
       }
       continue;
     }
 #pragma unroll
     for (uint32_t u = 0; u < (16u >> k); ++u) {
-      const uint32_t t = tw.t[16 - (32u >> k) + u];
+      const double t = (double)(k == 1 ? tw.t1[u >> 2][u & 3] : k == 2 ? tw.t2[u & 3] : k == 3 ? tw.t3[u & 1] : tw.t4);
 #pragma unroll
       for (uint32_t l = 0; l < (1u << k); ++l) {
         const uint32_t q = (u << (k + 1)) | l;
-        bfly<INV>(v[q], v[q | (1u << k)], t);
+        bfly_f64<INV>(w[q], w[q | (1u << k)], t, M);
       }
     }
   }
 }
 
-// The low stages with each workgroup looping over tiles of 2^15 values (output columns 16-byte
-// aligned): one workgroup per CU, whose LDS holds one such tile and no second. As soon as a tile's first round has gone to
-// LDS, the workgroup issues the first round's loads of its next tile, and computes and stores the
-// second and third rounds while they are in flight. Vector memory operations complete in issue
-// order, so every vector load a tile still waits for is issued before the prefetch: the rounds at
-// bits 5 and 10 take their twiddles through the scalar cache, and the per-lane twiddles of the
-// round at bit 0 are loaded ahead (the forward transform's last round: with the tile's own
-// prefetch; the inverse transform's first round: together with the next tile's values). The only
-// wait on a prefetch is then the next tile's first round.
-// The tiles are split into 8 contiguous ranges, one per XCD (workgroup n runs on XCD n mod 8), and
-// the workgroups of an XCD take its tiles in turn: tiles of one column run side by side on one XCD
-// and share its L2. Every branch on `more` is uniform over the workgroup, so all waves meet the
-// same barriers and leave the loop together.
-// The looping kernel's first round (peeled off its loop: inside the loop, the round's waits for
-// the prefetch then have one path, after the previous tile's stores, and leave those in flight).
-template <bool INV, int S>
-__device__ __forceinline__ void loop_first_round(uint32_t* v, const Round0Tw& tw, uint32_t* lds, uint32_t gbase,
-                                                 const uint32_t* __restrict__ tree, uint32_t tree_len, uint32_t log_n) {
-  constexpr int A1 = INV ? 0 : 10, R1 = INV ? 5 : S - 10;
-  if constexpr (INV) round0_butterflies_pre<true>(v, tw);
-  else round_butterflies<false, S, A1, R1>(v, gbase, tree, tree_len, log_n);
-  round_to_lds<S, A1, R1>(v, lds);
+// F64_ROUND31 in a vector register: a fused multiply-add takes one scalar operand, the twiddle.
+__device__ __forceinline__ double round31_reg() {
+  double M = F64_ROUND31;
+  asm volatile("" : "+v"(M));
+  return M;
 }
 
-// 4 waves per SIMD: one 2^15 tile (1024 threads) per CU.
+// The kernel loops over tiles. A wave ends only when its stores are done, so with one tile per
+// workgroup the stores of a CU's tiles held its slots (1264 columns of 2^15 onto 2^16: 205 us). In the
+// loop a tile's loads are issued ahead of the previous tile's stores; vector memory operations complete
+// in issue order, so the wait for the loads leaves the stores in flight, and both pass under the other
+// waves' arithmetic: 184 us (the 32-bit kernel of before, its loads prefetched into registers: 243).
+// Bound by the VALU: about 1870 issue slots per lane and tile of 2^15, 157 us of these 184 with loads
+// and stores left out.
+//
+// The tiles are split into 8 contiguous ranges, one per XCD, and the workgroups of an XCD take its
+// tiles in turn, so all waves of a workgroup meet the same barriers. 4 waves per SIMD: LDS holds 2^15
+// values (and their padding), 32 a lane.
 template <bool INV, int S>
-__global__ void __launch_bounds__(LowShape<S>::T, 4) fft_low_loop_kernel(const uint32_t* const* __restrict__ src,
-                                                                      uint32_t* const* __restrict__ dst, uint32_t log_n,
-                                                                      uint32_t in_mask, const uint32_t* __restrict__ tree,
-                                                                      uint32_t tree_len, uint32_t scale, uint32_t prio,
-                                                                      uint32_t n_tiles) {
+__global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* const* __restrict__ src,
+                                                              uint32_t* const* __restrict__ dst, uint32_t log_n,
+                                                              uint32_t in_mask, const uint32_t* __restrict__ t_end,
+                                                              const double* __restrict__ td_end, uint32_t rot,
+                                                              uint32_t prio, uint32_t n_tiles) {
   if (prio) CRITICAL_PATH_WAVE();
   constexpr uint32_t N = 1u << S;
-  // rounds in execution order: the inverse runs bits 0-4, 5-9, 10..S-1; the forward the reverse
-  constexpr int A1 = INV ? 0 : 10, R1 = INV ? 5 : S - 10;
-  constexpr int A3 = INV ? 10 : 0, R3 = INV ? S - 10 : 5;
-  __shared__ uint32_t lds[N + (N >> 5)];
-  const uint32_t per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7;
-  const uint32_t t_end = (uint32_t)(((uint64_t)n_tiles * (xcd + 1)) >> 3);
-  uint32_t tile = (uint32_t)(((uint64_t)n_tiles * xcd) >> 3) + (blockIdx.x >> 3);
-  if (tile >= t_end) return;
+  __shared__ __align__(16) uint32_t lds[N + (N >> 5)];
+  __shared__ double tw5[TW5_STRIDE * (LOW_T<S> >> 5)];
+  const bool split = (gridDim.x & 7) == 0;
+  const uint32_t step = split ? gridDim.x >> 3 : gridDim.x, xcd = blockIdx.x & 7;
+  const uint32_t tile_end = split ? (uint32_t)(((uint64_t)n_tiles * (xcd + 1)) >> 3) : n_tiles;
+  uint32_t tile = split ? (uint32_t)(((uint64_t)n_tiles * xcd) >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  if (tile >= tile_end) return;
   const uint32_t blk_log = log_n - S, blk_mask = (1u << blk_log) - 1;
-  uint32_t v[LowShape<S>::V], w[LowShape<S>::V];
-  Round0Tw tw;  // the round at bit 0: the inverse's first (next tile's), the forward's last
-  {
-    const GLOBAL_AS uint32_t* __restrict__ in = gmem(src[tile >> blk_log]);
-    round_from_global<S, A1, R1>(v, in, (tile & blk_mask) << S, in_mask, (reinterpret_cast<uintptr_t>(in) & 15) == 0);
-    if constexpr (INV) load_round0_tw<S>(tw, (tile & blk_mask) << S, tree, tree_len, log_n);
-    loop_first_round<INV, S>(v, tw, lds, (tile & blk_mask) << S, tree, tree_len, log_n);
-  }
-  for (;;) {
+  const double M = round31_reg();
+  // The previous tile's results: the inverse's in r, the forward's in LDS. Before the first tile the
+  // stores run all the same, to a buffer of no words, which drops them: on a second path without them
+  // the compiler could not count the stores that its waits may leave in flight.
+  uint32_t r[32];
+#pragma unroll
+  for (uint32_t i = 0; i < 32; ++i) r[i] = 0;
+  GLOBAL_AS uint32_t* out = gmem(dst[tile >> blk_log]);
+  uint32_t out_words = 0;
+  const auto store = [&](uint32_t t) {
+    if constexpr (INV) store_round10<S>(r, out, out_words, t);
+    else store_round0(lds, out, out_words, t);
+  };
+  for (;; tile += step) {
     const uint32_t gbase = (tile & blk_mask) << S;
-    if constexpr (!INV) load_round0_tw<S>(tw, gbase, tree, tree_len, log_n);
-    const uint32_t next = tile + per_xcd;
-    const bool more = next < t_end;
-    {
-      // v is free: the next tile's first-round values (the last tile loads its own again, unused:
-      // a branch here would make the compiler's waits below cover the prefetch)
-      const uint32_t pf = more ? next : tile;
-      const GLOBAL_AS uint32_t* __restrict__ nin = gmem(src[pf >> blk_log]);
-      round_from_global<S, A1, R1>(v, nin, (pf & blk_mask) << S, in_mask, (reinterpret_cast<uintptr_t>(nin) & 15) == 0);
-      if constexpr (INV) load_round0_tw<S>(tw, (pf & blk_mask) << S, tree, tree_len, log_n);
+    const GLOBAL_AS uint32_t* in = gmem(src[tile >> blk_log]) + (gbase & in_mask);  // in_mask >= 2^S - 1
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // keeps the lane's addresses out of registers between the tiles
+    double w[32];
+    uint32_t v[32];
+    Round0Tw tw;
+    if constexpr (INV) {
+      load_round0(v, in, t);
+      load_round0_tw(tw, gbase, t_end, log_n, t);
+    } else {
+      load_round10<S>(v, in, t);
     }
-    // the loads above stay here: the compiler may not sink them past this point
-    asm volatile("" ::: "memory");
-    __syncthreads();
-    round_from_lds<S, 5, 5>(w, lds);
-    round_butterflies<INV, S, 5, 5>(w, gbase, tree, tree_len, log_n);
-    round_to_lds<S, 5, 5>(w, lds);
-    __syncthreads();
-    round_from_lds<S, A3, R3>(w, lds);
-    if constexpr (INV) round_butterflies<true, S, A3, R3>(w, gbase, tree, tree_len, log_n);
-    else round0_butterflies_pre<false>(w, tw);
-    GLOBAL_AS uint32_t* __restrict__ out = gmem(dst[tile >> blk_log]);
-    // one store path (the launch requires 16-byte aligned output columns): with two, the compiler
-    // could not tell how many stores are in flight when the next tile's first round waits
-    round_to_global<S, A3, R3, true>(w, out, gbase, scale, true, 1u << log_n);
-    if (!more) break;
-    __syncthreads();  // this tile's last LDS reads end before the next tile's first writes
-    tile = next;
-    loop_first_round<INV, S>(v, tw, lds, (tile & blk_mask) << S, tree, tree_len, log_n);
+    const double tw5_in = load_tw5(gbase, td_end, log_n, t);
+    asm volatile("" ::: "memory");  // the loads stay ahead of the stores
+    store(t);
+    to_f64(w, v);
+    store_tw5(tw5, tw5_in, t);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (INV) {
+      round0_butterflies<true>(w, tw, M);
+      __syncthreads();  // the last tile's reads in the round at bit 10 are done
+      round_to_lds<S, 0, 5>(w, lds, t);
+      wave_lds_fence();
+      __builtin_amdgcn_sched_barrier(0);
+      round_from_lds<S, 5, 5>(w, lds, t);
+      round5_butterflies<true>(w, tw5, M, t);
+      round_to_lds<S, 5, 5>(w, lds, t);
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+      round_from_lds<S, 10, S - 10>(w, lds, t);
+      round10_butterflies<true, S, S - 10>(w, gbase, td_end, log_n, M);
+      canon_words(r, w, rot);
+    } else {
+      round10_butterflies<false, S, S - 10>(w, gbase, td_end, log_n, M);
+      __syncthreads();  // the last tile's words have left LDS
+      round_to_lds<S, 10, S - 10>(w, lds, t);
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+      load_round0_tw(tw, gbase, t_end, log_n, t);
+      round_from_lds<S, 5, 5>(w, lds, t);
+      round5_butterflies<false>(w, tw5, M, t);
+      round_to_lds<S, 5, 5>(w, lds, t);
+      wave_lds_fence();
+      __builtin_amdgcn_sched_barrier(0);
+      round_from_lds<S, 0, 5>(w, lds, t);
+      round0_butterflies<false>(w, tw, M);
+      round0_stage_out(w, lds, t);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    out = gmem(dst[tile >> blk_log]) + gbase;
+    out_words = N;
+    if (tile + step >= tile_end) return store(t);
   }
 }
 
-template <bool INV>
-static void launch_low_loop(uint32_t S, uint32_t n_cols, const uint32_t* const* src, uint32_t* const* dst,
-                            uint32_t log_n, uint32_t in_mask, const uint32_t* tree, uint32_t tree_len, uint32_t scale,
-                            uint32_t prio, hipStream_t stream) {
+// Foreground transforms run as many workgroups as the device holds at once, each looping over tiles;
+// a background one has a workgroup per tile, so that the kernels beside it get CUs as its tiles end (a
+// grid that holds every CU until the transform is done doubled the time of the trace's Merkle tree).
+template <bool INV, int S>
+static void launch_low_tile(uint32_t n_cols, const uint32_t* const* src, uint32_t* const* dst, uint32_t log_n,
+                            uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
   int dev = 0, cus = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const uint32_t n_tiles = n_cols << (log_n - S);
-  // one workgroup per CU (its LDS holds one 2^15 tile), a multiple of 8 (the XCD split), no more
-  // than the tiles
-  uint32_t n_wg = (uint32_t)cus / 8 * 8;
-  if (n_wg < 8) n_wg = 8;
-  while (n_wg > 8 && n_wg > n_tiles) n_wg -= 8;
-  const dim3 grid(n_wg), block(1u << (S - 5));
-  hipLaunchKernelGGL((fft_low_loop_kernel<INV, 15>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale,
-                     prio, n_tiles);
+  const uint32_t n_tiles = n_cols << (log_n - S), resident = (uint32_t)(cus > 8 ? cus / 8 * 8 : 8) << (15 - S);
+  const uint32_t grid = prio && n_tiles > resident ? resident : n_tiles;
+  hipLaunchKernelGGL((fft_low_kernel<INV, S>), dim3(grid), dim3(LOW_T<S>), 0, stream, src, dst, log_n, in_mask,
+                     tree.t + tree.len, tree.td_end, rot, prio, n_tiles);
 }
-
 template <bool INV>
 static void launch_low(uint32_t S, uint32_t n_cols, const uint32_t* const* src, uint32_t* const* dst, uint32_t log_n,
-                       uint32_t in_mask, const uint32_t* tree, uint32_t tree_len, uint32_t scale, uint32_t prio,
-                       hipStream_t stream) {
-  const dim3 grid(n_cols << (log_n - S)), block(1u << (S - 5));
+                       uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
   switch (S) {
-    case 11: hipLaunchKernelGGL((fft_low_kernel<INV, 11>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale, prio); break;
-    case 12: hipLaunchKernelGGL((fft_low_kernel<INV, 12>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale, prio); break;
-    case 13: hipLaunchKernelGGL((fft_low_kernel<INV, 13>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale, prio); break;
-    case 14: hipLaunchKernelGGL((fft_low_kernel<INV, 14>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale, prio); break;
-    default: hipLaunchKernelGGL((fft_low_kernel<INV, 15>), grid, block, 0, stream, src, dst, log_n, in_mask, tree, tree_len, scale, prio); break;
+    case 11: return launch_low_tile<INV, 11>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
+    case 12: return launch_low_tile<INV, 12>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
+    case 13: return launch_low_tile<INV, 13>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
+    case 14: return launch_low_tile<INV, 14>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
+    default: return launch_low_tile<INV, 15>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
   }
 }
 
@@ -587,10 +565,11 @@ static std::vector<FftPass> plan_passes(uint32_t k, uint32_t K) {
 }
 
 void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,
-                uint32_t log_n, const uint32_t* tree, uint32_t tree_len, hipStream_t stream, bool background,
-                uint32_t low_log) {
+                uint32_t log_n, const FftTree& ft, hipStream_t stream, bool background, uint32_t low_log) {
   if (n_cols == 0) return;
   const uint32_t prio = background ? 0u : 1u;
+  const uint32_t* const tree = ft.t2;
+  const uint32_t tree_len = ft.len;
   const uint32_t k = inverse ? log_n : log_in;  // number of stages actually run
   const uint32_t inv_n = inverse ? 2 * m31_inv(1u << log_n) : 0;  // doubled, as the twiddles
   auto run_pass = [&](const FftPass& ps, const uint32_t* const* from, uint32_t mask, uint32_t scale) {
@@ -629,7 +608,7 @@ void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, 
     low_log &= ~FFT_LOW_LOOP;
     if (low_log != 0 && (low_log < 11 || low_log > smax)) throw std::invalid_argument("launch_fft: low_log out of range");
     const uint32_t S = low_log ? low_log : smax;
-    if (loop && S != 15) throw std::invalid_argument("launch_fft: the looping low kernel needs low_log 15");
+    if (loop && S != 15) throw std::invalid_argument("launch_fft: FFT_LOW_LOOP needs low_log 15");
     // the stages above the low tile: register passes of at most PASS_REG_MAX stages, as even as
     // the count allows (8 stages: 4 + 4, not 6 + 2)
     std::vector<FftPass> high;
@@ -641,19 +620,17 @@ void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, 
         e += st;
       }
     }
-    auto low = [&](bool inv, const uint32_t* const* from, uint32_t mask, uint32_t scale) {
-      if (inv) (loop ? launch_low_loop<true> : launch_low<true>)(S, n_cols, from, dst, log_n, mask, tree, tree_len, scale, prio, stream);
-      else (loop ? launch_low_loop<false> : launch_low<false>)(S, n_cols, from, dst, log_n, mask, tree, tree_len, scale, prio, stream);
-    };
     if (inverse) {
-      low(true, src, full, high.empty() ? inv_n : 0u);
+      // 2^-log_n is 2^(31 - log_n): the low stages' own scaling is a rotation
+      launch_low<true>(S, n_cols, src, dst, log_n, full, ft, high.empty() ? 31 - log_n : 0u, prio, stream);
       for (size_t i = 0; i < high.size(); ++i)
         run_pass(high[i], (const uint32_t* const*)dst, full, i + 1 == high.size() ? inv_n : 0u);
     } else {
       for (size_t ii = high.size(); ii-- > 0;)
         run_pass(high[ii], ii + 1 == high.size() ? src : (const uint32_t* const*)dst,
                  ii + 1 == high.size() ? in_mask : full, 0u);
-      low(false, high.empty() ? src : (const uint32_t* const*)dst, high.empty() ? in_mask : full, 0u);
+      launch_low<false>(S, n_cols, high.empty() ? src : (const uint32_t* const*)dst, dst, log_n,
+                        high.empty() ? in_mask : full, ft, 0u, prio, stream);
     }
     return;
   }

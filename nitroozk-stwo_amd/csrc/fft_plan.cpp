@@ -8,19 +8,14 @@
 // workgroups than the device has CUs, or ends in a partly filled wave of workgroups. A smaller
 // tile spreads the same transform over more workgroups, at the cost of one more pass over HBM.
 //
-// The low stages of 2^15-value tiles can also run in a looping kernel (FFT_LOW_LOOP): one
-// workgroup per CU, loading its next tile while it computes the current one, which hides the loads
-// of a tile that no second workgroup on the CU could overlap. It writes 16 bytes at a time, so a plan
-// that uses it is only taken for 16-byte aligned output columns (Ctx::fft_plan_for).
-//
-// The autotuner times every candidate (each S, and the looping kernel at S = 15) once per
-// (device, direction, columns, sizes) on scratch columns and keeps the fastest; transforms of at
-// most 15 stages whose largest-tile grid fills the device four times over take S = k without
-// timing (looping when forward and S = 15), larger ones are timed on a subset of their columns.
-// A transform beside critical-path work on another stream is planned, and timed, without the
-// looping kernel: its workgroups would hold every CU until the transform ends. Choices persist across processes in the cache directory as
-// fft_plans_<arch>_<CUs>.txt, one "direction n_cols log_in log_n plan" line per shape (direction: 1
-// for inverse, plus 2 for a background transform; plan: S, plus 256 for the looping kernel).
+// The autotuner times every candidate S once per (device, direction, foreground or background,
+// columns, sizes) on scratch columns and keeps the fastest; transforms of at most 15 stages whose
+// largest-tile grid fills the device four times over take S = k without timing (with the flag
+// FFT_LOW_LOOP when forward and S = 15, as plans of that shape always had; launch_fft does the same with
+// and without it), larger ones are timed on a subset of their columns. Choices persist across processes
+// in the cache directory as fft_plans_<arch>_<CUs>_f64.txt (the name changes with the kernels that were
+// timed), one "direction n_cols log_in log_n plan" line per shape (direction: 1 for inverse, plus 2 for
+// a background transform; plan: S, plus 256 for the flag).
 // STWO_HIP_FFT_TUNE=0 turns the timing off (a fixed rule picks S instead).
 #include <fcntl.h>
 #include <sys/stat.h>
@@ -62,7 +57,7 @@ std::string plan_file(int device, int cus) {
   if (hipGetDeviceProperties(&prop, device) != hipSuccess) return {};
   std::string arch = prop.gcnArchName;
   if (auto c = arch.find(':'); c != std::string::npos) arch.resize(c);
-  return d + "/fft_plans_" + arch + "_" + std::to_string(cus) + ".txt";
+  return d + "/fft_plans_" + arch + "_" + std::to_string(cus) + "_f64.txt";
 }
 
 // With g_mu held.
@@ -102,15 +97,8 @@ bool tuning_enabled() {
 
 }  // namespace
 
-uint32_t Ctx::fft_plan_for(uint32_t plan, uint32_t* const* dst, size_t n_cols) {
-  if (plan & FFT_LOW_LOOP)
-    for (size_t c = 0; c < n_cols; ++c)
-      if (reinterpret_cast<uintptr_t>(dst[c]) & 15) return plan & ~FFT_LOW_LOOP;
-  return plan;
-}
-
-uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const uint32_t* tree2,
-                          uint32_t tree_len, bool background) {
+uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree,
+                          bool background) {
   const uint32_t k = inverse ? log_n : log_in;
   if (k < 11 || n_cols == 0) return 0;
   const uint32_t smax = k < 15 ? k : 15;
@@ -123,8 +111,8 @@ uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32
   if (smax == 11) return smax;
   const bool fills = ((uint64_t)n_cols << (log_n - smax)) >= 4 * cus;
   // transforms of at most 15 stages that fill the device four times over: one pass of the largest
-  // tile, for forward transforms in the looping kernel, whose workgroups load their next tile while
-  // they compute (the inverse gains nothing from it)
+  // tile (1264 columns of 2^15 onto 2^16: 187 us against 252 to 309 with smaller tiles and a strided pass;
+  // the inverse 117 against 142 to 153)
   if (fills && k <= 15) return smax | (!inverse && !background && smax == 15 ? FFT_LOW_LOOP : 0u);
   const PlanKey key{device, (inverse ? 1u : 0u) + (background ? 2u : 0u), n_cols, log_in, log_n};
   {
@@ -151,24 +139,22 @@ uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32
   HIP_CHECK(hipMallocFromPoolAsync((void**)&dst, (size_t)n_cols * out_words * 4, pool, stream));
   launch_fill_zero(src, (size_t)n_cols * in_words, stream);
   std::vector<const uint32_t*> s_tab(n_cols);
-  std::vector<uint32_t*> d_tab(n_cols);  // 256-byte aligned blocks: every candidate applies
+  std::vector<uint32_t*> d_tab(n_cols);
   for (uint32_t c = 0; c < n_cols; ++c) {
     s_tab[c] = src + (size_t)c * in_words;
     d_tab[c] = dst + (size_t)c * out_words;
   }
   const auto* ds = (const uint32_t* const*)upload_vec(s_tab);
   auto* dd = (uint32_t* const*)upload_vec(d_tab);
-  // candidates: every tile, and the looping kernel with 2^15 values
   std::vector<uint32_t> cand;
   for (uint32_t s = 11; s <= smax; ++s) cand.push_back(s);
-  if (smax == 15 && !background) cand.push_back(15 | FFT_LOW_LOOP);
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
   for (uint32_t c : cand) {
-    launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree2, tree_len, stream, false, c);  // warm-up
+    launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, stream, background, c);  // warm-up
     for (int rep = 0; rep < 2; ++rep) {
       hipEvent_t a = get_event(), b = get_event();
       HIP_CHECK(hipEventRecord(a, stream));
-      launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree2, tree_len, stream, false, c);
+      launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, stream, background, c);
       HIP_CHECK(hipEventRecord(b, stream));
       ev.push_back({a, b});
     }

@@ -12,16 +12,24 @@ struct Cols4 { uint32_t* c[4]; };
 struct CCols4 { const uint32_t* c[4]; };
 
 // fft.hip
-// tree: a doubled twiddle tree (every entry 2t; Ctx::tw2 for evaluation, Ctx::itw2 for
-// interpolation). background: the transform runs beside critical-path kernels on another stream
-// and leaves them the issue priority. low_log: the tile of the low-stage kernel, 2^low_log values
-// per workgroup (11 <= low_log <= min(k, 15) for a transform of k >= 11 stages; 0 = the largest),
-// the stages above it run in strided passes. low_log | FFT_LOW_LOOP (low_log 15; every output
-// column 16-byte aligned): the low-stage kernel runs one workgroup per CU, each looping over tiles
-// and loading its next tile while it computes the current one.
+// A twiddle tree as the transforms read it (the inverse tree for interpolation): len entries t, the
+// same doubled (t2), and the end of the table of its last max(1, len / 16) entries as doubles (the
+// stages from 5 on).
+struct FftTree {
+  const uint32_t* t;
+  const uint32_t* t2;
+  const double* td_end;
+  uint32_t len;
+};
+inline size_t fft_tree_doubles(size_t len) { return len < 16 ? 1 : len / 16; }
+// background: the transform runs beside critical-path kernels on another stream and leaves them the
+// issue priority, and CUs as its tiles end. low_log: the tile of the low-stage kernel, 2^low_log values
+// per workgroup (11 <= low_log <= min(k, 15) for a transform of k >= 11 stages; 0 = the largest), the
+// stages above it run in strided passes. FFT_LOW_LOOP may be set on top of 15; foreground transforms loop
+// over their tiles with any low_log, so it changes nothing.
 constexpr uint32_t FFT_LOW_LOOP = 0x100;
 void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,
-                uint32_t log_n, const uint32_t* tree, uint32_t tree_len, hipStream_t stream, bool background = false,
+                uint32_t log_n, const FftTree& tree, hipStream_t stream, bool background = false,
                 uint32_t low_log = 0);
 
 // merkle.hip
@@ -267,7 +275,7 @@ struct GenPowers { cpm31 p[31]; };
 // (2^log_size words each); zero_flag (one word, cleared by the caller) is raised when an
 // x-coordinate is zero.
 void launch_twiddle_tree(uint32_t init_index, uint32_t log_size, uint32_t* tw, uint32_t* itw, uint32_t* tw2,
-                         uint32_t* itw2, uint32_t* zero_flag, hipStream_t stream);
+                         uint32_t* itw2, double* twd, double* itwd, uint32_t* zero_flag, hipStream_t stream);
 void launch_bit_reverse(uint32_t* col, uint32_t log_n, hipStream_t stream);
 // Circle transforms on domains of log size 1 or 2 (the half coset's first point given).
 void launch_fft_tiny(bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,

@@ -5,10 +5,11 @@
 // v_alignbit_b32 (the operations of a Blake2s round), written one instruction per asm statement so
 // that the count is exact: 24 VALU instructions per loop iteration and lane.
 //
-// butterfly_kernel: every lane holds 32 M31 values in registers and runs rounds of 5 butterfly
-// stages on them (80 butterflies per round), with the FFT's own butterfly code (butterfly.h) and
-// twiddles held in registers: the rate of the transform's arithmetic with no memory traffic, the
-// ceiling of the FFT kernels' butterflies per second.
+// butterfly_kernel: every lane holds 32 M31 values in registers, as doubles, and runs rounds of 5
+// butterfly stages on them (80 butterflies per round), with the FFT's own code (butterfly.h: the
+// butterflies, and the packing and unpacking of every value between two rounds) and twiddles held in
+// registers: the rate of the transform's arithmetic with no memory traffic, the ceiling of the FFT
+// kernels' butterflies per second.
 //
 // compression_kernel: every lane holds a Blake2s chaining state and a 64-byte message block in
 // registers and compresses with the Merkle kernels' own one-lane code (blake2s.h), each result
@@ -68,29 +69,33 @@ double measure_int32_issue(uint32_t* scratch, hipStream_t stream) {
 
 template <bool INV>
 __global__ void __launch_bounds__(256) butterfly_kernel(uint32_t iters, uint32_t seed, uint32_t* out) {
-  uint32_t v[32], tw[16];
+  double v[32], tw[16];
+  double M = F64_ROUND31;
+  asm volatile("" : "+v"(M));
 #pragma unroll
-  for (int k = 0; k < 32; ++k) v[k] = (seed * (threadIdx.x + 1) + 7919u * k) & P;
+  for (int k = 0; k < 32; ++k) v[k] = (double)((seed * (threadIdx.x + 1) + 7919u * k) & P);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) tw[k] = 2u * ((seed * 2654435761u + 40503u * k + threadIdx.x) & 0x3fffffffu);
+  for (int k = 0; k < 16; ++k) tw[k] = (double)((seed * 2654435761u + 40503u * k + threadIdx.x) & 0x3fffffffu);
   for (uint32_t it = 0; it < iters; ++it) {
 #pragma unroll
     for (int kk = 0; kk < 5; ++kk) {
       const int k = INV ? kk : 4 - kk;  // the FFT's stage order within a round
 #pragma unroll
       for (int u = 0; u < (32 >> (k + 1)); ++u) {
-        const uint32_t t = tw[(u + 3 * k) & 15];
+        const double t = tw[(u + 3 * k) & 15];
 #pragma unroll
         for (int l = 0; l < (1 << k); ++l) {
           const int q = (u << (k + 1)) | l;
-          bfly<INV>(v[q], v[q | (1 << k)], t);
+          bfly_f64<INV>(v[q], v[q | (1 << k)], t, M);
         }
       }
     }
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k] = (double)pack_f64(v[k]);  // as between the transforms' rounds
   }
   uint32_t s = 0;
 #pragma unroll
-  for (int k = 0; k < 32; ++k) s ^= v[k];
+  for (int k = 0; k < 32; ++k) s ^= pack_f64(v[k]);
   if (s == 0x12345678u) out[blockIdx.x] = s;  // keeps the values live
 }
 

@@ -245,9 +245,7 @@ void evaluate_into(Ctx& ctx, const std::vector<const uint32_t*>& coeffs, const s
     }
     const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
     uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
-    const uint32_t low = Ctx::fft_plan_for(
-        ctx.fft_low_log(false, (uint32_t)idx.size(), lg, target_log, ctx.tw2.p, ctx.tree_len(), on_side), dst.data(),
-        dst.size());
+    const uint32_t low = ctx.fft_low_log(false, (uint32_t)idx.size(), lg, target_log, ctx.fft_tree(false), on_side);
     hipStream_t st = ctx.stream;
     if (on_side) {
       ctx.fork();  // the side stream starts after the upload and everything queued before it
@@ -255,7 +253,7 @@ void evaluate_into(Ctx& ctx, const std::vector<const uint32_t*>& coeffs, const s
     }
     KScope ks(ctx, K_EVALUATE, (double)idx.size() * (4.0 * (1u << lg) + 4.0 * (1u << target_log)), st);
     ks.units(fft_butterflies(idx.size(), target_log, lg));
-    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, target_log, ctx.tw2.p, ctx.tree_len(), st, on_side, low);
+    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, target_log, ctx.fft_tree(false), st, on_side, low);
   }
 }
 
@@ -399,11 +397,10 @@ void interpolate_columns(Ctx& ctx, const std::vector<const uint32_t*>& evals, co
     }
     const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
     uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
-    const uint32_t low = Ctx::fft_plan_for(ctx.fft_low_log(true, (uint32_t)idx.size(), lg, lg, ctx.itw2.p, ctx.tree_len()),
-                                           dst.data(), dst.size());
+    const uint32_t low = ctx.fft_low_log(true, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true));
     KScope ks(ctx, K_INTERPOLATE, (double)idx.size() * 8.0 * (1u << lg));
     ks.units(fft_butterflies(idx.size(), lg, lg));
-    launch_fft(true, d_src, d_dst, (uint32_t)idx.size(), lg, lg, ctx.itw2.p, ctx.tree_len(), ctx.stream, false, low);
+    launch_fft(true, d_src, d_dst, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true), ctx.stream, false, low);
   }
 }
 
@@ -429,11 +426,10 @@ void evaluate_polynomials(Ctx& ctx, DevTree& t, uint32_t log_blowup) {
     }
     const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
     uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
-    const uint32_t low = Ctx::fft_plan_for(ctx.fft_low_log(false, (uint32_t)idx.size(), lg, K, ctx.tw2.p, ctx.tree_len()),
-                                           dst.data(), dst.size());
+    const uint32_t low = ctx.fft_low_log(false, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false));
     KScope ks(ctx, K_EVALUATE, (double)idx.size() * (4.0 * (1u << lg) + 4.0 * (1u << K)));
     ks.units(fft_butterflies(idx.size(), K, lg));
-    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, K, ctx.tw2.p, ctx.tree_len(), ctx.stream, false, low);
+    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false), ctx.stream, false, low);
   }
 }
 

@@ -85,6 +85,8 @@ Ctx::~Ctx() {
   itw.reset();
   tw2.reset();
   itw2.reset();
+  twd.reset();
+  itwd.reset();
   domain_points.clear();
   fri_tickets.reset();
   gather_buf.reset();
@@ -337,7 +339,7 @@ void Ctx::d2h(void* dst, const void* src, size_t bytes) {
 // device (one lane per entry: the point by the generator's powers, the inverse by Fermat), so
 // that a tree of 2^29 entries costs milliseconds instead of a serial host loop.
 void build_twiddle_tree(Ctx& c, uint32_t init_index, uint32_t log_size, DevBuf& tw, DevBuf& itw, DevBuf& tw2,
-                        DevBuf& itw2) {
+                        DevBuf& itw2, DevBuf& twd, DevBuf& itwd) {
   if (log_size > 30) throw HipError(3, "coset log size must be at most 30");
   PersistentAllocScope keep(c);
   const size_t len = (size_t)1 << log_size;
@@ -345,8 +347,11 @@ void build_twiddle_tree(Ctx& c, uint32_t init_index, uint32_t log_size, DevBuf& 
   itw = DevBuf(&c, len);
   tw2 = DevBuf(&c, len);
   itw2 = DevBuf(&c, len);
+  twd = DevBuf(&c, 2 * fft_tree_doubles(len));
+  itwd = DevBuf(&c, 2 * fft_tree_doubles(len));
   DevBuf flag(&c, 1, true);
-  launch_twiddle_tree(init_index, log_size, tw.p, itw.p, tw2.p, itw2.p, flag.p, c.stream);
+  launch_twiddle_tree(init_index, log_size, tw.p, itw.p, tw2.p, itw2.p, (double*)twd.p, (double*)itwd.p,
+                      flag.p, c.stream);
   uint32_t zero = 0;
   c.d2h(&zero, flag.p, 4);
   if (zero) throw HipError(1, "the coset has a point with x = 0, whose twiddle has no inverse");
@@ -357,7 +362,7 @@ void build_twiddle_tree(Ctx& c, uint32_t init_index, uint32_t log_size, DevBuf& 
 void Ctx::ensure_twiddles(uint32_t log_domain) {
   if (log_domain <= tw_log) return;
   const uint32_t R = log_domain - 1;  // root coset log size
-  build_twiddle_tree(*this, HCoset::half_odds(R).initial_index, R, tw, itw, tw2, itw2);
+  build_twiddle_tree(*this, HCoset::half_odds(R).initial_index, R, tw, itw, tw2, itw2, twd, itwd);
   tw_log = log_domain;
 }
 

@@ -57,6 +57,11 @@ struct DevBuf {
   }
 };
 
+// A twiddle tree's buffers as the transforms read them (td: two words per double).
+inline FftTree make_fft_tree(const DevBuf& t, const DevBuf& t2, const DevBuf& td) {
+  return {t.p, t2.p, (const double*)td.p + td.n / 2, (uint32_t)t.n};
+}
+
 using Hash = std::array<uint8_t, 32>;
 
 struct StageTimes {
@@ -111,6 +116,8 @@ struct Ctx {
   uint32_t tw_log = 0;
   DevBuf tw, itw;
   DevBuf tw2, itw2;  // the same trees with every entry doubled (2t < 2^32), read by the FFT kernels
+  DevBuf twd, itwd;  // their last entries as doubles (FftTree), read by the FFT's low stages
+  FftTree fft_tree(bool inverse) const { return make_fft_tree(inverse ? itw : tw, inverse ? itw2 : tw2, inverse ? itwd : twd); }
   std::map<uint32_t, DevBuf> domain_points;  // bit-reversed (x, y) of CanonicCoset(log)
   // Ticket counters of the fused FRI layer launches, one per layer: zeroed once here, and every
   // launch leaves its counter at zero again.
@@ -170,14 +177,10 @@ struct Ctx {
   void ensure_twiddles(uint32_t log_domain);
   // Circle-FFT launch plans (fft_plan.cpp): the low-stage tile (2^S values per workgroup) for a
   // transform shape, as launch_fft's low_log; 0 for transforms of fewer than 11 stages. background:
-  // the transform runs beside critical-path kernels on another stream, and its plan leaves out the
-  // looping kernel (whose workgroups would hold every CU until the transform ends).
-  uint32_t fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const uint32_t* tree2,
-                       uint32_t tree_len, bool background = false);
+  // the transform runs beside critical-path kernels on another stream (planned and timed as such).
+  uint32_t fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree,
+                       bool background = false);
   uint32_t fft_low_override = 0;  // a fixed tile for every shape (stwo_hip_set_fft_low_log); 0 = planned
-  // The plan for output columns `dst` (host copies of their addresses): without the looping kernel
-  // unless every column is 16-byte aligned.
-  static uint32_t fft_plan_for(uint32_t plan, uint32_t* const* dst, size_t n_cols);
   int cu_count = 0;
   const uint32_t* domain_xy(uint32_t log);
   uint32_t tree_len() const { return 1u << (tw_log - 1); }
@@ -263,9 +266,10 @@ struct UploadBatch {
   ~UploadBatch() { if (!committed) c.commit_staged(); }
 };
 
-// The twiddle tree of Coset::new(init_index, log_size), plain and doubled (2^log_size words each).
+// The twiddle tree of Coset::new(init_index, log_size), plain and doubled (2^log_size words each), and
+// its last entries as doubles.
 void build_twiddle_tree(Ctx& c, uint32_t init_index, uint32_t log_size, DevBuf& tw, DevBuf& itw, DevBuf& tw2,
-                        DevBuf& itw2);
+                        DevBuf& itw2, DevBuf& twd, DevBuf& itwd);
 
 // ---- host Blake2s and channel ------------------------------------------------------------
 struct Blake2sHost {
