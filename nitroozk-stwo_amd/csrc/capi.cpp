@@ -89,10 +89,18 @@ void reject_unsatisfied(const stwo_proof& p) {
 // domains of log size 1 and 2 by the explicit formulas, larger ones by the FFT kernels over a
 // doubled tree whose last 2^(log_n - 1) entries are the domain's line twiddles.
 // `low` is the plan's low-stage tile (Ctx::fft_low_log), taken before the caller's timing scope.
-void run_fft(Ctx& c, bool inverse, const uint32_t* const* ds, uint32_t* const* dd, uint32_t n_cols, uint32_t log_in,
+void run_fft(Ctx& c, bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,
              uint32_t log_n, const FftTree& tree, uint32_t half_init, uint32_t low) {
-  if (log_n <= 2) launch_fft_tiny(inverse, ds, dd, n_cols, log_in, log_n, index_to_point(half_init), c.stream);
-  else launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, c.stream, false, low);
+  if (log_n <= 2) {
+    const auto* ds = (const uint32_t* const*)c.stage(src, n_cols * sizeof(*src));
+    auto* dd = (uint32_t* const*)c.stage(dst, n_cols * sizeof(*dst));
+    c.commit_staged();
+    launch_fft_tiny(inverse, ds, dd, n_cols, log_in, log_n, index_to_point(half_init), c.stream);
+    return;
+  }
+  const ColSet ds = c.col_set(src, n_cols, false), dd = c.col_set((const uint32_t* const*)dst, n_cols, false);
+  c.commit_staged();
+  launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, c.stream, false, low);
 }
 uint32_t plan_fft(Ctx& c, bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree) {
   return log_n <= 2 ? 0u : c.fft_low_log(inverse, n_cols, log_in, log_n, tree);
@@ -265,15 +273,11 @@ int stwo_hip_interpolate_columns(stwo_hip_ctx* h, const uint32_t* const* evals, 
   return guarded(h, [&](Ctx& c) {
     if (log_size < 1 || log_size > 30) throw HipError(3, "log_size must be in [1, 30]");
     c.ensure_twiddles(log_size < 2 ? 2 : log_size);
-    std::vector<const uint32_t*> s(evals, evals + n_cols);
-    std::vector<uint32_t*> d(coeffs, coeffs + n_cols);
-    const uint32_t* const* ds = (const uint32_t* const*)c.upload_vec(s);
-    uint32_t* const* dd = (uint32_t* const*)c.upload_vec(d);
     {
       const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, c.fft_tree(true));
       KScope ks(c, K_INTERPOLATE, (double)n_cols * 8.0 * (double)(1u << log_size));
       ks.units(fft_butterflies(n_cols, log_size, log_size));
-      run_fft(c, true, ds, dd, n_cols, log_size, log_size, c.fft_tree(true), canonic_half_init(log_size), low);
+      run_fft(c, true, evals, coeffs, n_cols, log_size, log_size, c.fft_tree(true), canonic_half_init(log_size), low);
     }
     c.end_stream_ordered();
   });
@@ -284,15 +288,11 @@ int stwo_hip_evaluate_polynomials(stwo_hip_ctx* h, const uint32_t* const* coeffs
     if (log_size < 1 || log_size + log_blowup > 30) throw HipError(3, "sizes out of range");
     const uint32_t log_n = log_size + log_blowup;
     c.ensure_twiddles(log_n < 2 ? 2 : log_n);
-    std::vector<const uint32_t*> s(coeffs, coeffs + n_cols);
-    std::vector<uint32_t*> d(evals, evals + n_cols);
-    const uint32_t* const* ds = (const uint32_t* const*)c.upload_vec(s);
-    uint32_t* const* dd = (uint32_t* const*)c.upload_vec(d);
     {
       const uint32_t low = plan_fft(c, false, n_cols, log_size, log_n, c.fft_tree(false));
       KScope ks(c, K_EVALUATE, (double)n_cols * (4.0 * (double)(1u << log_size) + 4.0 * (double)(1u << log_n)));
       ks.units(fft_butterflies(n_cols, log_n, log_size));
-      run_fft(c, false, ds, dd, n_cols, log_size, log_n, c.fft_tree(false), canonic_half_init(log_n), low);
+      run_fft(c, false, coeffs, evals, n_cols, log_size, log_n, c.fft_tree(false), canonic_half_init(log_n), low);
     }
     c.end_stream_ordered();
   });
@@ -314,8 +314,14 @@ int stwo_hip_batch_eval_at_point(stwo_hip_ctx* h, const uint32_t* const* coeffs,
     uint32_t max_chunks = oods_max_chunks(log_size);
     DevBuf partials(&c, (size_t)n_cols * max_chunks * 4), vals(&c, (size_t)n_cols * 4), w(&c, (size_t)4 << OODS_TABLE_LOG);
     const std::vector<uint32_t> bs = oods_batch_starts(tg);
-    launch_oods(c.upload_vec(tasks), c.upload_vec(tg), n_cols, c.upload_vec(bs), (uint32_t)bs.size() - 1, log_size,
-                c.upload_vec(f), c.upload_vec(gl), 1, (qm31*)w.p, (qm31*)partials.p, (qm31*)vals.p, c.stream);
+    const OodsTask* d_tasks = c.stage_vec(tasks);
+    const uint32_t* d_tg = c.stage_vec(tg);
+    const uint32_t* d_bs = c.stage_vec(bs);
+    const qm31* d_f = c.stage_vec(f);
+    const uint32_t* d_gl = c.stage_vec(gl);
+    c.commit_staged();
+    launch_oods(d_tasks, d_tg, n_cols, d_bs, (uint32_t)bs.size() - 1, log_size, d_f, d_gl, 1, (qm31*)w.p,
+                (qm31*)partials.p, (qm31*)vals.p, c.stream);
     c.d2h(out_host, vals.p, (size_t)n_cols * 16);
     c.reset_arena();
   });
@@ -418,15 +424,15 @@ int stwo_hip_commit_on_layer(stwo_hip_ctx* h, uint32_t log_size, const uint32_t*
     // columns laid out at a fixed stride of one column need no address table
     bool strided = n_cols > 1;
     for (uint32_t k = 1; strided && k < n_cols; ++k) strided = v[k] == v[0] + ((size_t)k << log_size);
-    // under graph capture, at most 16 columns travel as kernel arguments (no staged table)
-    const bool small = c.capturing && !strided;
-    if (small && n_cols > 16) throw HipError(3, "not capturable: more than 16 columns not at one stride");
-    const uint32_t* const* d = !strided && !small && n_cols ? (const uint32_t* const*)c.upload_vec(v) : nullptr;
+    // at most 16 columns travel as kernel arguments (no staged table; under graph capture the only way)
+    const bool small = n_cols <= 16;
+    if (c.capturing && !strided && !small) throw HipError(3, "not capturable: more than 16 columns not at one stride");
+    const uint32_t* const* d = !strided && !small ? (const uint32_t* const*)c.upload_vec(v) : nullptr;
     {
       KScope ks(c, K_MERKLE, ((prev ? 64.0 : 0.0) + 4.0 * n_cols + 32.0) * (double)(1u << log_size));
       ks.units(blake2s_node_compressions(prev != nullptr, n_cols) * (double)(1u << log_size));
-      if (strided) launch_merkle_layer_strided(log_size, prev, v[0], (size_t)1 << log_size, n_cols, out, c.stream);
-      else if (small) launch_merkle_layer_small(log_size, prev, v.data(), n_cols, out, c.stream);
+      if (small) launch_merkle_layer_small(log_size, prev, v.data(), n_cols, out, c.stream);
+      else if (strided) launch_merkle_layer_strided(log_size, prev, v[0], (size_t)1 << log_size, n_cols, out, c.stream);
       else launch_merkle_layer(log_size, prev, d, n_cols, out, c.stream);
     }
     c.end_stream_ordered();
@@ -500,9 +506,10 @@ int stwo_hip_fold_circle_into_line_grouped(stwo_hip_ctx* h, uint32_t log_src, ui
     if (aligned) {
       std::vector<const uint32_t*> sv(src, src + 4 * (size_t)n_groups);
       std::vector<uint32_t*> dv(dst, dst + 4 * (size_t)n_groups);
-      launch_fold_circle_into_line_grouped(log_src, n_groups, (const uint32_t* const*)c.upload_vec(sv),
-                                           (uint32_t* const*)c.upload_vec(dv), q(alpha), c.itw.p, c.tree_len(),
-                                           c.stream);
+      const auto* ds = (const uint32_t* const*)c.stage_vec(sv);
+      auto* dd = (uint32_t* const*)c.stage_vec(dv);
+      c.commit_staged();
+      launch_fold_circle_into_line_grouped(log_src, n_groups, ds, dd, q(alpha), c.itw.p, c.tree_len(), c.stream);
     } else {
       for (uint32_t g = 0; g < n_groups; ++g)
         launch_fold_circle_into_line(log_src, {{src[4 * g], src[4 * g + 1], src[4 * g + 2], src[4 * g + 3]}},
@@ -609,7 +616,10 @@ int stwo_hip_compute_quotients_and_combine(stwo_hip_ctx* h, const stwo_accumulat
       qp.part_end = (uint32_t)parts.size();
       pts.push_back(qp);
     }
-    launch_quotients(lifting_log_size, c.domain_xy(lifting_log_size), c.upload_vec(pts), n_accs, c.upload_vec(parts),
+    const QuotPoint* d_pts = c.stage_vec(pts);
+    const QuotPart* d_parts = c.stage_vec(parts);
+    c.commit_staged();
+    launch_quotients(lifting_log_size, c.domain_xy(lifting_log_size), d_pts, n_accs, d_parts,
                      {{out[0], out[1], out[2], out[3]}}, c.stream);
     c.end_stream_ordered();
   });
@@ -763,8 +773,11 @@ int stwo_hip_evaluate_constraint_quotients_on_domain(stwo_hip_ctx* h, uint32_t* 
     std::vector<const uint32_t*> tv(trace, trace + n_trace);
     if (id == fnv1a("fibonacci_example")) {
       if (n_trace < 2 || n_constraints != n_trace - 2) throw HipError(1, "wide-fib: n_constraints must be n_trace - 2");
-      launch_wide_fib_composition(eval_log, trace_log, (const uint32_t* const*)c.upload_vec(tv), n_trace,
-                                  c.upload_vec(pows), c.upload_vec(dinv), a4, true, c.stream);
+      const auto* d_t = (const uint32_t* const*)c.stage_vec(tv);
+      const qm31* d_w = c.stage_vec(pows);
+      const uint32_t* d_d = c.stage_vec(dinv);
+      c.commit_staged();
+      launch_wide_fib_composition(eval_log, trace_log, d_t, n_trace, d_w, d_d, a4, true, c.stream);
     } else if (id == fnv1a("poseidon_example")) {
       if (blob_len < 4 + 4 + 32) throw HipError(1, "poseidon eval_blob too short");
       PoseidonParams pp{};
@@ -779,9 +792,13 @@ int stwo_hip_evaluate_constraint_quotients_on_domain(stwo_hip_ctx* h, uint32_t* 
       for (int i = 0; i < 16; ++i) { pp.alpha_pow[i] = p; p = qm_mul(p, a); }
       pp.shift = q(cumsum_shift);
       std::vector<const uint32_t*> iv(interaction, interaction + n_interaction);
-      launch_poseidon_composition(eval_log, trace_log, (const uint32_t* const*)c.upload_vec(tv),
-                                  (const uint32_t* const*)c.upload_vec(iv), (const PoseidonParams*)c.upload(&pp, sizeof(pp)),
-                                  pp.ipr, c.upload_vec(pows), c.upload_vec(dinv), a4, true, c.stream);
+      const auto* d_t = (const uint32_t* const*)c.stage_vec(tv);
+      const auto* d_i = (const uint32_t* const*)c.stage_vec(iv);
+      const auto* d_p = (const PoseidonParams*)c.stage(&pp, sizeof(pp));
+      const qm31* d_w = c.stage_vec(pows);
+      const uint32_t* d_d = c.stage_vec(dinv);
+      c.commit_staged();
+      launch_poseidon_composition(eval_log, trace_log, d_t, d_i, d_p, pp.ipr, d_w, d_d, a4, true, c.stream);
     } else if (id == fnv1a("expr_component")) {
       // a constraint program, compiled into a kernel on first use: u32 program words, the
       // program, u32 parameter count, the parameters (QM31 each); parameter 0 is cumsum_shift
@@ -802,11 +819,12 @@ int stwo_hip_evaluate_constraint_quotients_on_domain(stwo_hip_ctx* h, uint32_t* 
       if (compiled_component_constraints(words.data(), words.size()) != n_constraints)
         throw HipError(1, "expr_component: n_constraints differs from the program's");
       std::vector<const uint32_t*> iv(interaction, interaction + n_interaction);
-      const auto* d_t = (const uint32_t* const*)c.upload_vec(tv);
-      const auto* d_i = n_interaction ? (const uint32_t* const*)c.upload_vec(iv) : nullptr;
-      const qm31* d_p = c.upload_vec(params);
-      const qm31* d_w = c.upload_vec(pows);
-      const uint32_t* d_d = c.upload_vec(dinv);
+      const auto* d_t = (const uint32_t* const*)c.stage_vec(tv);
+      const auto* d_i = n_interaction ? (const uint32_t* const*)c.stage_vec(iv) : nullptr;
+      const qm31* d_p = c.stage_vec(params);
+      const qm31* d_w = c.stage_vec(pows);
+      const uint32_t* d_d = c.stage_vec(dinv);
+      c.commit_staged();
       KScope ks(c, K_COMPOSITION, (4.0 * (n_trace + n_interaction) + 32.0) * (double)(1u << eval_log));
       evaluate_compiled_component(c.device, words.data(), words.size(), eval_log, trace_log, d_t, n_trace, d_i,
                                   n_interaction, d_p, (uint32_t)params.size(), d_w, n_constraints, d_d, a4, c.stream);
@@ -1163,13 +1181,11 @@ int stwo_hip_interpolate_on_domain(stwo_hip_ctx* h, const stwo_hip_twiddles* t, 
     if (!t || !h->trees.count(const_cast<stwo_hip_twiddles*>(t))) throw HipError(1, "unknown twiddle tree");
     check_tree(t, half_coset_initial_index, log_size);
     if (n_cols == 0) return;
-    std::vector<const uint32_t*> s(evals, evals + n_cols);
-    std::vector<uint32_t*> d(coeffs, coeffs + n_cols);
     {
       const uint32_t low = plan_fft(c, true, n_cols, log_size, log_size, t->fft_tree(true));
       KScope ks(c, K_INTERPOLATE, (double)n_cols * 8.0 * (double)(1u << log_size));
       ks.units(fft_butterflies(n_cols, log_size, log_size));
-      run_fft(c, true, (const uint32_t* const*)c.upload_vec(s), (uint32_t* const*)c.upload_vec(d), n_cols, log_size,
+      run_fft(c, true, evals, coeffs, n_cols, log_size,
               log_size, t->fft_tree(true), half_coset_initial_index, low);
     }
     c.end_stream_ordered();
@@ -1183,13 +1199,11 @@ int stwo_hip_evaluate_on_domain(stwo_hip_ctx* h, const stwo_hip_twiddles* t, uin
     check_tree(t, half_coset_initial_index, log_size);
     if (log_coeffs < 1 || log_coeffs > log_size) throw HipError(1, "coefficients larger than the domain");
     if (n_cols == 0) return;
-    std::vector<const uint32_t*> s(coeffs, coeffs + n_cols);
-    std::vector<uint32_t*> d(evals, evals + n_cols);
     {
       const uint32_t low = plan_fft(c, false, n_cols, log_coeffs, log_size, t->fft_tree(false));
       KScope ks(c, K_EVALUATE, (double)n_cols * (4.0 * (double)(1u << log_coeffs) + 4.0 * (double)(1u << log_size)));
       ks.units(fft_butterflies(n_cols, log_size, log_coeffs));
-      run_fft(c, false, (const uint32_t* const*)c.upload_vec(s), (uint32_t* const*)c.upload_vec(d), n_cols, log_coeffs,
+      run_fft(c, false, coeffs, evals, n_cols, log_coeffs,
               log_size, t->fft_tree(false), half_coset_initial_index, low);
     }
     c.end_stream_ordered();

@@ -19,6 +19,14 @@
 
 namespace sh {
 
+// Column c (the same for a whole workgroup) of a transform's columns.
+__device__ __forceinline__ const GLOBAL_AS uint32_t* col_in(const ColSet& s, uint32_t c) {
+  return gmem(s.table ? s.table[c] : s.base + (int64_t)c * s.step);
+}
+__device__ __forceinline__ GLOBAL_AS uint32_t* col_out(const ColSet& s, uint32_t c) {
+  return gmem(const_cast<uint32_t*>(s.table ? s.table[c] : s.base + (int64_t)c * s.step));
+}
+
 // Doubled circle twiddle of pair h (line layer 0 pairs [x, y] -> [y, -y, -x, x]).
 __device__ __forceinline__ uint32_t circle_twiddle(const uint32_t* __restrict__ lt0, uint32_t h) {
   const uint32_t x = lt0[(h >> 2) * 2], y = lt0[(h >> 2) * 2 + 1];
@@ -75,16 +83,15 @@ __device__ __forceinline__ void radix_round(uint32_t* lds, uint32_t C, uint32_t 
 }
 
 template <bool INV>
-__global__ void __launch_bounds__(256) fft_pass_kernel(const uint32_t* const* __restrict__ src,
-                                                       uint32_t* const* __restrict__ dst, uint32_t log_n,
+__global__ void __launch_bounds__(256) fft_pass_kernel(ColSet src, ColSet dst, uint32_t log_n,
                                                        uint32_t in_mask, uint32_t e, uint32_t S, uint32_t c,
                                                        const uint32_t* __restrict__ tree, uint32_t tree_len,
                                                        uint32_t scale, uint32_t prio) {
   if (prio) CRITICAL_PATH_WAVE();
   extern __shared__ uint32_t lds[];
   const uint32_t col = blockIdx.y;
-  const GLOBAL_AS uint32_t* __restrict__ in = gmem(src[col]);
-  GLOBAL_AS uint32_t* __restrict__ out = gmem(dst[col]);
+  const GLOBAL_AS uint32_t* __restrict__ in = col_in(src, col);
+  GLOBAL_AS uint32_t* __restrict__ out = col_out(dst, col);
   const uint32_t C = 1u << c;
   const uint32_t tile = blockIdx.x;
   const uint32_t lo_blk = tile & ((1u << (e - c)) - 1);
@@ -121,15 +128,14 @@ __global__ void __launch_bounds__(256) fft_pass_kernel(const uint32_t* const* __
 // wave, and every twiddle (index (hi 2^(S-1-j)) + (t >> (j + 1)) at stage e + j) is the same for the
 // whole wave: a scalar load. No LDS and no barrier.
 template <bool INV, int S>
-__global__ void __launch_bounds__(256) fft_pass_reg_kernel(const uint32_t* const* __restrict__ src,
-                                                           uint32_t* const* __restrict__ dst, uint32_t log_n,
+__global__ void __launch_bounds__(256) fft_pass_reg_kernel(ColSet src, ColSet dst, uint32_t log_n,
                                                            uint32_t in_mask, uint32_t e,
                                                            const uint32_t* __restrict__ tree, uint32_t tree_len,
                                                            uint32_t scale, uint32_t prio) {
   if (prio) CRITICAL_PATH_WAVE();
   const uint32_t col = blockIdx.y;
-  const GLOBAL_AS uint32_t* __restrict__ in = gmem(src[col]);
-  GLOBAL_AS uint32_t* __restrict__ out = gmem(dst[col]);
+  const GLOBAL_AS uint32_t* __restrict__ in = col_in(src, col);
+  GLOBAL_AS uint32_t* __restrict__ out = col_out(dst, col);
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t lo = g & ((1u << e) - 1);
   const uint32_t hi = __builtin_amdgcn_readfirstlane(g >> e);  // e >= 6: one value per wave
@@ -431,8 +437,7 @@ __device__ __forceinline__ double round31_reg() {
 // tiles in turn, so all waves of a workgroup meet the same barriers. 4 waves per SIMD: LDS holds 2^15
 // values (and their padding), 32 a lane.
 template <bool INV, int S>
-__global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* const* __restrict__ src,
-                                                              uint32_t* const* __restrict__ dst, uint32_t log_n,
+__global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(ColSet src, ColSet dst, uint32_t log_n,
                                                               uint32_t in_mask, const uint32_t* __restrict__ t_end,
                                                               const double* __restrict__ td_end, uint32_t rot,
                                                               uint32_t prio, uint32_t n_tiles) {
@@ -453,7 +458,7 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* co
   uint32_t r[32];
 #pragma unroll
   for (uint32_t i = 0; i < 32; ++i) r[i] = 0;
-  GLOBAL_AS uint32_t* out = gmem(dst[tile >> blk_log]);
+  GLOBAL_AS uint32_t* out = col_out(dst, tile >> blk_log);
   uint32_t out_words = 0;
   const auto store = [&](uint32_t t) {
     if constexpr (INV) store_round10<S>(r, out, out_words, t);
@@ -461,7 +466,7 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* co
   };
   for (;; tile += step) {
     const uint32_t gbase = (tile & blk_mask) << S;
-    const GLOBAL_AS uint32_t* in = gmem(src[tile >> blk_log]) + (gbase & in_mask);  // in_mask >= 2^S - 1
+    const GLOBAL_AS uint32_t* in = col_in(src, tile >> blk_log) + (gbase & in_mask);  // in_mask >= 2^S - 1
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));  // keeps the lane's addresses out of registers between the tiles
     double w[32];
@@ -510,7 +515,7 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* co
       round0_stage_out(w, lds, t);
     }
     __builtin_amdgcn_sched_barrier(0);
-    out = gmem(dst[tile >> blk_log]) + gbase;
+    out = col_out(dst, tile >> blk_log) + gbase;
     out_words = N;
     if (tile + step >= tile_end) return store(t);
   }
@@ -520,7 +525,7 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(const uint32_t* co
 // a background one has a workgroup per tile, so that the kernels beside it get CUs as its tiles end (a
 // grid that holds every CU until the transform is done doubled the time of the trace's Merkle tree).
 template <bool INV, int S>
-static void launch_low_tile(uint32_t n_cols, const uint32_t* const* src, uint32_t* const* dst, uint32_t log_n,
+static void launch_low_tile(uint32_t n_cols, ColSet src, ColSet dst, uint32_t log_n,
                             uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
   int dev = 0, cus = 0;
   (void)hipGetDevice(&dev);
@@ -531,7 +536,7 @@ static void launch_low_tile(uint32_t n_cols, const uint32_t* const* src, uint32_
                      tree.t + tree.len, tree.td_end, rot, prio, n_tiles);
 }
 template <bool INV>
-static void launch_low(uint32_t S, uint32_t n_cols, const uint32_t* const* src, uint32_t* const* dst, uint32_t log_n,
+static void launch_low(uint32_t S, uint32_t n_cols, ColSet src, ColSet dst, uint32_t log_n,
                        uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
   switch (S) {
     case 11: return launch_low_tile<INV, 11>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
@@ -564,7 +569,7 @@ static std::vector<FftPass> plan_passes(uint32_t k, uint32_t K) {
   return p;
 }
 
-void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,
+void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t log_in,
                 uint32_t log_n, const FftTree& ft, hipStream_t stream, bool background, uint32_t low_log) {
   if (n_cols == 0) return;
   const uint32_t prio = background ? 0u : 1u;
@@ -572,7 +577,7 @@ void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, 
   const uint32_t tree_len = ft.len;
   const uint32_t k = inverse ? log_n : log_in;  // number of stages actually run
   const uint32_t inv_n = inverse ? 2 * m31_inv(1u << log_n) : 0;  // doubled, as the twiddles
-  auto run_pass = [&](const FftPass& ps, const uint32_t* const* from, uint32_t mask, uint32_t scale) {
+  auto run_pass = [&](const FftPass& ps, const ColSet& from, uint32_t mask, uint32_t scale) {
     if (ps.c == ~0u) {  // a register pass (after the low stages: e >= 11, 2^(log_n - S) >= 256 lanes)
       const dim3 grid(1u << (log_n - ps.S - 8), n_cols), block(256);
 #define PASS_REG(SS)                                                                                            \
@@ -624,12 +629,12 @@ void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, 
       // 2^-log_n is 2^(31 - log_n): the low stages' own scaling is a rotation
       launch_low<true>(S, n_cols, src, dst, log_n, full, ft, high.empty() ? 31 - log_n : 0u, prio, stream);
       for (size_t i = 0; i < high.size(); ++i)
-        run_pass(high[i], (const uint32_t* const*)dst, full, i + 1 == high.size() ? inv_n : 0u);
+        run_pass(high[i], dst, full, i + 1 == high.size() ? inv_n : 0u);
     } else {
       for (size_t ii = high.size(); ii-- > 0;)
-        run_pass(high[ii], ii + 1 == high.size() ? src : (const uint32_t* const*)dst,
+        run_pass(high[ii], ii + 1 == high.size() ? src : dst,
                  ii + 1 == high.size() ? in_mask : full, 0u);
-      launch_low<false>(S, n_cols, high.empty() ? src : (const uint32_t* const*)dst, dst, log_n,
+      launch_low<false>(S, n_cols, high.empty() ? src : dst, dst, log_n,
                         high.empty() ? in_mask : full, ft, 0u, prio, stream);
     }
     return;
@@ -637,11 +642,11 @@ void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, 
   auto passes = plan_passes(k, log_n);
   if (inverse) {
     for (size_t i = 0; i < passes.size(); ++i)
-      run_pass(passes[i], i == 0 ? src : (const uint32_t* const*)dst, full, i + 1 == passes.size() ? inv_n : 0u);
+      run_pass(passes[i], i == 0 ? src : dst, full, i + 1 == passes.size() ? inv_n : 0u);
   } else {
     for (size_t ii = passes.size(); ii-- > 0;) {
       const bool first = ii + 1 == passes.size();
-      run_pass(passes[ii], first ? src : (const uint32_t* const*)dst, first ? in_mask : full, 0u);
+      run_pass(passes[ii], first ? src : dst, first ? in_mask : full, 0u);
     }
   }
 }

@@ -138,14 +138,7 @@ uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32
   HIP_CHECK(hipMallocFromPoolAsync((void**)&src, (size_t)n_cols * in_words * 4, pool, stream));
   HIP_CHECK(hipMallocFromPoolAsync((void**)&dst, (size_t)n_cols * out_words * 4, pool, stream));
   launch_fill_zero(src, (size_t)n_cols * in_words, stream);
-  std::vector<const uint32_t*> s_tab(n_cols);
-  std::vector<uint32_t*> d_tab(n_cols);
-  for (uint32_t c = 0; c < n_cols; ++c) {
-    s_tab[c] = src + (size_t)c * in_words;
-    d_tab[c] = dst + (size_t)c * out_words;
-  }
-  const auto* ds = (const uint32_t* const*)upload_vec(s_tab);
-  auto* dd = (uint32_t* const*)upload_vec(d_tab);
+  const ColSet ds{nullptr, src, (int64_t)in_words}, dd{nullptr, dst, (int64_t)out_words};
   std::vector<uint32_t> cand;
   for (uint32_t s = 11; s <= smax; ++s) cand.push_back(s);
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;

@@ -28,9 +28,15 @@ inline size_t fft_tree_doubles(size_t len) { return len < 16 ? 1 : len / 16; }
 // stages above it run in strided passes. FFT_LOW_LOOP may be set on top of 15; foreground transforms loop
 // over their tiles with any low_log, so it changes nothing.
 constexpr uint32_t FFT_LOW_LOOP = 0x100;
-void launch_fft(bool inverse, const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_in,
-                uint32_t log_n, const FftTree& tree, hipStream_t stream, bool background = false,
-                uint32_t low_log = 0);
+// The columns of a transform: a device table of addresses, or (null table) column c at base + c step
+// words, which needs no table at all.
+struct ColSet {
+  const uint32_t* const* table;
+  const uint32_t* base;
+  int64_t step;
+};
+void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
+                const FftTree& tree, hipStream_t stream, bool background = false, uint32_t low_log = 0);
 
 // merkle.hip
 void launch_merkle_layer(uint32_t log_size, const uint32_t* prev, const uint32_t* const* cols, uint32_t n_cols,
@@ -265,6 +271,10 @@ void launch_poseidon_logup_fracs(uint32_t log_n, uint32_t ipr, const uint32_t* c
 void launch_coset_prefix_sum(uint32_t log_n, uint32_t* const* cols4, qm31 shift, const unsigned long long* shift_sums,
                              uint32_t* scratch, hipStream_t stream);
 
+// `bytes` (at most sizeof(StageArgs)) from host memory to dst as a launch's arguments, in stream order:
+// the host memory is free on return.
+struct StageArgs { uint32_t w[896]; };
+void launch_stage_args(uint32_t* dst, const void* src, size_t bytes, hipStream_t stream);
 void launch_fill_zero(uint32_t* p, size_t n, hipStream_t stream);
 void launch_copy_words(uint32_t* dst, const uint32_t* src, size_t n, hipStream_t stream);
 

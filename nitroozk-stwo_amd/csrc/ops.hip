@@ -7,6 +7,8 @@
 //   lift_and_accumulate    prover/backend/cpu/accumulation.rs (lifted index (i >> (r+1) << 1) + (i & 1))
 //   eval_at_point          prover/backend/cpu/circle.rs:82-99; core/poly/utils.rs:27-70
 // All kernels are HBM streaming kernels: one lane per row, coordinate columns read coalesced.
+#include <cstring>
+#include <stdexcept>
 #include "field.h"
 #include "kernels.h"
 
@@ -812,6 +814,17 @@ void launch_decommit_gather(const DecItem* items, uint32_t n_items, const uint32
     for (uint32_t i = 0; i < q.n; ++i) q.p[i] = positions[f + i];
     hipLaunchKernelGGL(decommit_gather_kernel, dim3(n_items, q.n), dim3(256), 0, stream, items, q, out);
   }
+}
+
+// Words that travel as kernel arguments, written to device memory.
+__global__ void __launch_bounds__(256) stage_args_kernel(StageArgs a, uint32_t n, uint32_t* __restrict__ dst) {
+  for (uint32_t i = threadIdx.x; i < n; i += 256) gmem(dst)[i] = a.w[i];
+}
+void launch_stage_args(uint32_t* dst, const void* src, size_t bytes, hipStream_t stream) {
+  if (bytes > sizeof(StageArgs)) throw std::invalid_argument("launch_stage_args: more than an argument block holds");
+  StageArgs a;
+  std::memcpy(a.w, src, bytes);
+  hipLaunchKernelGGL(stage_args_kernel, dim3(1), dim3(256), 0, stream, a, (uint32_t)((bytes + 3) / 4), dst);
 }
 
 __global__ void fill_zero_kernel(uint32_t* p, size_t n) {

@@ -243,8 +243,7 @@ void evaluate_into(Ctx& ctx, const std::vector<const uint32_t*>& coeffs, const s
       src.push_back(coeffs[i]);
       dst.push_back(out[i].p);
     }
-    const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
-    uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
+    const ColSet d_src = ctx.col_set(src, true), d_dst = ctx.col_set(dst, true);
     const uint32_t low = ctx.fft_low_log(false, (uint32_t)idx.size(), lg, target_log, ctx.fft_tree(false), on_side);
     hipStream_t st = ctx.stream;
     if (on_side) {
@@ -395,8 +394,7 @@ void interpolate_columns(Ctx& ctx, const std::vector<const uint32_t*>& evals, co
       into.coeffs[base + i] = dst.back();
       into.coeff_logs[base + i] = lg;
     }
-    const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
-    uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
+    const ColSet d_src = ctx.col_set(src, true), d_dst = ctx.col_set(dst, true);
     const uint32_t low = ctx.fft_low_log(true, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true));
     KScope ks(ctx, K_INTERPOLATE, (double)idx.size() * 8.0 * (1u << lg));
     ks.units(fft_butterflies(idx.size(), lg, lg));
@@ -424,8 +422,7 @@ void evaluate_polynomials(Ctx& ctx, DevTree& t, uint32_t log_blowup) {
       t.evals[i] = dst.back();
       t.eval_logs[i] = K;
     }
-    const uint32_t* const* d_src = (const uint32_t* const*)ctx.table_vec(src);
-    uint32_t* const* d_dst = (uint32_t* const*)ctx.table_vec(dst);
+    const ColSet d_src = ctx.col_set(src, true), d_dst = ctx.col_set(dst, true);
     const uint32_t low = ctx.fft_low_log(false, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false));
     KScope ks(ctx, K_EVALUATE, (double)idx.size() * (4.0 * (1u << lg) + 4.0 * (1u << K)));
     ks.units(fft_butterflies(idx.size(), K, lg));

@@ -133,12 +133,25 @@ void* Ctx::stage(const void* src, size_t bytes) {
   return d;
 }
 void Ctx::commit_staged() {
-  if (pinned_off > staged_from) {
-    HIP_CHECK(hipMemcpyAsync(dev_arena + staged_from, pinned + staged_from, pinned_off - staged_from,
+  const size_t n = pinned_off - staged_from;
+  if (n && n <= sizeof(StageArgs)) {
+    // small tables ride in a launch's arguments: a queued copy of the same bytes cost the host and the
+    // stream more, and holds the pinned bytes until it is done
+    launch_stage_args((uint32_t*)(dev_arena + staged_from), pinned + staged_from, n, stream);
+  } else if (n) {
+    HIP_CHECK(hipMemcpyAsync(dev_arena + staged_from, pinned + staged_from, n,
                              hipMemcpyHostToDevice, stream));
     uploads_in_flight = true;
   }
   staged_from = pinned_off;
+}
+ColSet Ctx::col_set(const uint32_t* const* cols, size_t n, bool keep) {
+  const intptr_t step = n > 1 ? (intptr_t)cols[1] - (intptr_t)cols[0] : 0;
+  bool even = step % 4 == 0;
+  for (size_t k = 2; even && k < n; ++k) even = (intptr_t)cols[k] - (intptr_t)cols[k - 1] == step;
+  if (even) return {nullptr, n ? cols[0] : nullptr, (int64_t)(step / 4)};
+  const size_t bytes = n * sizeof(*cols);
+  return {(const uint32_t* const*)(keep ? upload_table(cols, bytes) : stage(cols, bytes)), nullptr, 0};
 }
 void* Ctx::col_alloc(size_t bytes) {
   bytes = (bytes + 255) & ~(size_t)255;

@@ -158,6 +158,11 @@ struct Ctx {
   // table goes to a buffer of its own, with the same lifetime.
   const void* upload_table(const void* src, size_t bytes);
   template <class T> const T* table_vec(const std::vector<T>& v) { return (const T*)upload_table(v.data(), v.size() * sizeof(T)); }
+  // A transform's columns: at one distance from each other (the rows of one allocation), else by a table,
+  // staged (valid once commit_staged() has queued it) or kept (as upload_table).
+  ColSet col_set(const uint32_t* const* cols, size_t n, bool keep);
+  ColSet col_set(const std::vector<const uint32_t*>& v, bool keep) { return col_set(v.data(), v.size(), keep); }
+  ColSet col_set(const std::vector<uint32_t*>& v, bool keep) { return col_set((const uint32_t* const*)v.data(), v.size(), keep); }
   struct TableEntry { size_t off, bytes; };
   std::unordered_multimap<uint64_t, TableEntry> table_cache;  // content hash -> table in table_dev
   uint8_t* table_dev = nullptr;
