@@ -627,8 +627,9 @@ int stwo_hip_compute_quotients_and_combine(stwo_hip_ctx* h, const stwo_accumulat
 
 int stwo_hip_accumulate(stwo_hip_ctx* h, uint32_t log_size, uint32_t* const dst[4], const uint32_t* const src[4]) {
   return guarded(h, [&](Ctx& c) {
-    launch_accumulate_lifted(log_size, {{dst[0], dst[1], dst[2], dst[3]}}, log_size, {{src[0], src[1], src[2], src[3]}},
-                             c.stream);
+    const LiftSource s{{src[0], src[1], src[2], src[3]}, log_size};
+    launch_accumulate_lifts(log_size, {{dst[0], dst[1], dst[2], dst[3]}}, {{dst[0], dst[1], dst[2], dst[3]}}, &s, 1,
+                            c.stream);
     c.end_stream_ordered();
   });
 }
@@ -640,11 +641,12 @@ int stwo_hip_lift_and_accumulate(stwo_hip_ctx* h, const uint32_t* const* cols4, 
       if (log_sizes[i] < log_sizes[i - 1]) throw HipError(1, "columns must be sorted by increasing size");
     if (log_sizes[0] < 1) throw HipError(1, "A column must be of length at least 2.");
     uint32_t L = log_sizes[n_cols - 1];
-    Cols4 o = {{out[0], out[1], out[2], out[3]}};
-    for (int k = 0; k < 4; ++k) launch_copy_words(out[k], cols4[4 * (n_cols - 1) + k], (size_t)1 << L, c.stream);
+    const uint32_t* const* top = cols4 + 4 * (size_t)(n_cols - 1);
+    std::vector<LiftSource> s(n_cols - 1);
     for (uint32_t i = 0; i + 1 < n_cols; ++i)
-      launch_accumulate_lifted(L, o, log_sizes[i], {{cols4[4 * i], cols4[4 * i + 1], cols4[4 * i + 2], cols4[4 * i + 3]}},
-                               c.stream);
+      s[i] = LiftSource{{cols4[4 * i], cols4[4 * i + 1], cols4[4 * i + 2], cols4[4 * i + 3]}, log_sizes[i]};
+    launch_accumulate_lifts(L, {{out[0], out[1], out[2], out[3]}}, {{top[0], top[1], top[2], top[3]}}, s.data(), s.size(),
+                            c.stream);
     c.end_stream_ordered();
   });
 }

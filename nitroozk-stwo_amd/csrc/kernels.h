@@ -149,7 +149,12 @@ void launch_quotient_coeffs(qm31 qrc, const qm31* vals, const QCoefEntry* entrie
 void launch_quotients(uint32_t lifting_log, const uint32_t* domain_xy, const QuotPoint* points, uint32_t n_points,
                       const QuotPart* parts, Cols4 out, hipStream_t stream);
 
-void launch_accumulate_lifted(uint32_t log_dst, Cols4 dst, uint32_t log_src, CCols4 src, hipStream_t stream);
+// dst = base + the lifts of the sources (at most 2^log_dst rows each) to 2^log_dst rows; base may be dst.
+struct LiftSource { const uint32_t* c[4]; uint32_t log_size; };
+constexpr uint32_t LIFT_ARGS = 24;  // sources per launch
+struct LiftArgs { struct { const uint32_t* c[4]; uint32_t r; } s[LIFT_ARGS]; };
+void launch_accumulate_lifts(uint32_t log_dst, Cols4 dst, CCols4 base, const LiftSource* src, size_t n_src,
+                             hipStream_t stream);
 
 // OODS: value of FFT-basis coefficient columns at QM31 points. Tasks are grouped by (point, size):
 // group_factors[g*32 + b] is the folding factor of bit b (y, x, pi(x), ...). Scratch: weights holds

@@ -688,8 +688,11 @@ int prove_ex(Ctx& ctx, Channel& ch, std::vector<DevTree>& trees, const std::vect
   // finalize: lift smaller accumulations into the largest, then interpolate 4 coordinate columns
   auto& big = accs[max_log];
   Cols4 b4 = {{big[0].p, big[1].p, big[2].p, big[3].p}};
+  std::vector<LiftSource> lifts;
   for (auto& [lg, a] : accs)
-    if (lg != max_log) launch_accumulate_lifted(max_log, b4, lg, {{a[0].p, a[1].p, a[2].p, a[3].p}}, ctx.stream);
+    if (lg != max_log) lifts.push_back(LiftSource{{a[0].p, a[1].p, a[2].p, a[3].p}, lg});
+  if (!lifts.empty())
+    launch_accumulate_lifts(max_log, b4, {{b4.c[0], b4.c[1], b4.c[2], b4.c[3]}}, lifts.data(), lifts.size(), ctx.stream);
   HMARK("x_compkernel");
   DevTree comp;
   {
