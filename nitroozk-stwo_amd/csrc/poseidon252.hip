@@ -10,6 +10,7 @@
 // one permutation per two absorbed values (214 Montgomery products), so the kernel is VALU-bound.
 #include <stdexcept>
 #include "felt252.h"
+#include "felt252_rows.h"
 #include "kernels.h"
 
 namespace sh {
@@ -52,6 +53,50 @@ __global__ void __launch_bounds__(256) p252_layer_kernel(uint32_t n, const uint3
   for (int j = 0; j < 8; ++j) out[8 * (size_t)i + j] = r.w[j];
 }
 
+// The same layer with a node on the 16 lanes of a row (felt252_rows.h), four nodes to a wave: for layers
+// of few nodes, which wait for one permutation whatever their size.
+__device__ const RowTable ROW_TABLE = make_row_table();
+__global__ void __launch_bounds__(64) p252_rows_kernel(uint32_t n, const uint32_t* __restrict__ prev,
+                                                       const uint32_t* const* __restrict__ cols, uint32_t n_cols,
+                                                       uint32_t* __restrict__ out) {
+  __shared__ int32_t tab[ROWS_N * 16];
+  for (uint32_t j = threadIdx.x; j < ROWS_N * 16; j += 64) tab[j] = ROW_TABLE.v[j];
+  __syncthreads();
+  const uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 4);
+  if (i >= n) return;  // whole rows
+  const Row R(tab, threadIdx.x & 15);
+  int32_t s[3] = {0, 0, 0};
+  if (prev && n_cols == 0) {
+    s[0] = R.to_mont(R.limb_at(prev + 16 * (size_t)i));
+    s[1] = R.to_mont(R.limb_at(prev + 16 * (size_t)i + 8));
+    s[2] = R.at(ROWS_TWO);
+    R.permute(s);
+  } else {
+    // poseidon_hash_many: the two children (if any), then the columns' values packed 8 to a felt252; a pair
+    // of absorbed values and a permutation at a time, the last with the padding 1
+    const uint32_t n_felts = (prev ? 2u : 0u) + (n_cols + 7) / 8;
+    const auto felt = [&](uint32_t j) -> int32_t {
+      if (prev && j < 2) return R.to_mont(R.limb_at(prev + 16 * (size_t)i + 8 * j));
+      const uint32_t c0 = 8 * (j - (prev ? 2u : 0u)), m = n_cols - c0 < 8 ? n_cols - c0 : 8;
+      uint32_t x[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (uint32_t q = 0; q < m; ++q) x[q] = gmem(cols[c0 + q])[i];
+      return R.to_mont(R.limb_of(felt_from_m31s(x, (int)m)));
+    };
+#pragma unroll 1
+    for (uint32_t j = 0; j <= n_felts; j += 2) {
+      const int32_t one = R.at(ROWS_ONE);
+      s[0] = R.carry(s[0] + (j < n_felts ? felt(j) : one));
+      if (j < n_felts) s[1] = R.carry(s[1] + (j + 1 < n_felts ? felt(j + 1) : one));
+      R.permute(s);
+    }
+  }
+  const F r = R.from_mont(s[0]);
+  if ((threadIdx.x & 15) == 0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) gmem(out)[8 * (size_t)i + j] = r.w[j];
+  }
+}
+
 // Nonces (hi << 32) | lo with lo < 2^14 (GRIND_LOW_BITS of prover/backend/simd/grind.rs:150-190),
 // candidate j of the launch at hi = hi0 + j / 2^14: a hash of (prefixed digest, nonce) with pow_bits
 // trailing zero bits (of its low 128 bits, as u128::trailing_zeros of the big-endian bytes 16..32)
@@ -85,9 +130,15 @@ __global__ void __launch_bounds__(256) p252_perm_rate_kernel(uint32_t iters, uin
 
 }  // namespace
 
+// Layers of at most 2^P252_ROWS_LOG nodes run on rows.
+constexpr uint32_t P252_ROWS_LOG = 13;
 void launch_p252_layer(uint32_t log_size, const uint32_t* prev, const uint32_t* const* cols, uint32_t n_cols,
                        uint32_t* out, hipStream_t stream) {
   const uint32_t n = 1u << log_size;
+  if (log_size <= P252_ROWS_LOG) {
+    hipLaunchKernelGGL(p252_rows_kernel, dim3((n + 3) / 4), dim3(64), 0, stream, n, prev, cols, n_cols, out);
+    return;
+  }
   hipLaunchKernelGGL(p252_layer_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, n, prev, cols, n_cols, out);
 }
 
