@@ -215,7 +215,11 @@ int stwo_hip_copy_h2d(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_
   });
 }
 int stwo_hip_copy_d2h(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_t n) {
-  return guarded(h, [&](Ctx& c) { c.d2h(dst, src, n * 4); });
+  return guarded(h, [&](Ctx& c) {
+    // memory that is not a whole column of this context (any other is the copy engine's to judge)
+    const auto it = c.col_live.find(const_cast<uint32_t*>(src));
+    c.d2h(dst, src, n * 4, it != c.col_live.end() && it->second >= n * 4);
+  });
 }
 static_assert(GATHER_ARG_COLS * GATHER_ARG_ROWS <= Ctx::gather_host_words,
               "an argument-block gather must fit the coherent host buffer");
@@ -232,8 +236,9 @@ int stwo_hip_batch_at_multi(stwo_hip_ctx* h, const uint32_t* const* cols, uint32
       GatherArgs g{};
       for (uint32_t k = 0; k < n_cols; ++k) g.cols[k] = cols[k];
       for (uint32_t r = 0; r < n_rows; ++r) g.rows[r] = rows[r];
-      launch_gather_args(g, n_cols, n_rows, c.gather_host_dev, true, c.stream);
-      c.sync_main();
+      c.commit_staged();
+      launch_gather_args(g, n_cols, n_rows, c.gather_host_dev, c.gather_flag(), ++c.gather_call, c.stream);
+      c.wait_gather();
       std::memcpy(out_host, c.gather_host, n * 4);
       c.reset_arena();
       return;

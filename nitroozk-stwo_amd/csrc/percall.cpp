@@ -640,6 +640,8 @@ int prove_ex(const Api& a, typename MC::Ch& ch, std::vector<Tree>& trees, const 
     out.commitments.push_back(t.root);
   }
 
+  a.ck(stwo_hip_synchronize(a.h), "synchronize");  // what the calls have left to the runtime is not the caller's
+
   // ---- sanity check (prover/mod.rs:127-144) ----
   const size_t lt = S.n_trees() - 1;
   const qm31 lft = from_partial_evals(S.vals(lt, 0)[0], S.vals(lt, 1)[0], S.vals(lt, 2)[0], S.vals(lt, 3)[0]);

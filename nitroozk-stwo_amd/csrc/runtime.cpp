@@ -1,6 +1,7 @@
 // Host runtime of libstwo_hip (see runtime.h).
 #include "runtime.h"
 #include <cstring>
+#include <chrono>
 #include <cstdlib>
 
 #include <algorithm>
@@ -71,7 +72,9 @@ Ctx::Ctx(int dev) : device(dev) {
   pinned_cap = 64u << 20;
   HIP_CHECK(hipHostMalloc((void**)&pinned, pinned_cap, hipHostMallocDefault));
   HIP_CHECK(hipHostMalloc((void**)&d2h_pinned, d2h_cap, hipHostMallocDefault));
-  HIP_CHECK(hipHostMalloc((void**)&gather_host, gather_host_words * 4, hipHostMallocCoherent | hipHostMallocMapped));
+  HIP_CHECK(hipHostMalloc((void**)&gather_host, (gather_host_words + 16) * 4,
+                          hipHostMallocCoherent | hipHostMallocMapped));
+  gather_host[gather_host_words] = gather_call;
   HIP_CHECK(hipHostGetDevicePointer((void**)&gather_host_dev, gather_host, 0));
   arena_cap = 64u << 20;
   HIP_CHECK(hipMalloc((void**)&dev_arena, arena_cap));
@@ -277,6 +280,24 @@ void Ctx::sync_main() {
   commit_staged();
   HIP_CHECK(hipStreamSynchronize(stream));
   uploads_in_flight = false;
+  polls = 0;
+}
+void Ctx::wait_gather() {
+  const uint32_t* flag = gather_host + gather_host_words;
+  if (++polls < GATHER_POLLS) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(GATHER_POLL_US);
+    do {
+      for (int i = 0; i < 64; ++i) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == gather_call) {
+          uploads_in_flight = false;  // queued before the gather
+          return;
+        }
+        __builtin_ia32_pause();
+      }
+    } while (std::chrono::steady_clock::now() < until);
+  }
+  sync_main();
+  if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != gather_call) throw HipError(1, "a gather did not complete");
 }
 void Ctx::sync() {
   commit_staged();
@@ -284,6 +305,7 @@ void Ctx::sync() {
   side_busy = false;
   HIP_CHECK(hipStreamSynchronize(stream));
   uploads_in_flight = false;
+  polls = 0;
   // event pairs are folded into kstats in bulk (each elapsed-time query costs host time)
   if (pending.size() >= 16384) collect_timing();
 }
@@ -334,7 +356,15 @@ void* Ctx::readback_buf(size_t bytes) {
   }
   return rb_pinned;
 }
-void Ctx::d2h(void* dst, const void* src, size_t bytes) {
+void Ctx::d2h(void* dst, const void* src, size_t bytes, bool by_kernel) {
+  if (by_kernel && bytes && bytes <= READ_WORDS * 4 && (bytes | (uintptr_t)src) % 4 == 0) {
+    commit_staged();
+    launch_read_words((const uint32_t*)src, (uint32_t)(bytes / 4), gather_host_dev, gather_flag(), ++gather_call,
+                      stream);
+    wait_gather();
+    std::memcpy(dst, gather_host, bytes);
+    return;
+  }
   // through pinned memory: a read-back into pageable memory goes through the runtime's own
   // staging, which costs tens of microseconds more per call
   if (bytes <= d2h_cap) {

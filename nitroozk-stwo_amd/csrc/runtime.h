@@ -189,12 +189,27 @@ struct Ctx {
   int cu_count = 0;
   const uint32_t* domain_xy(uint32_t log);
   uint32_t tree_len() const { return 1u << (tw_log - 1); }
-  void d2h(void* dst, const void* src, size_t bytes);  // synchronous
-  // Coherent pinned host memory that small gathers write directly from the device (zero copy; the
-  // kernel ends with a system-scope fence, the host reads after the stream synchronises).
+  // Synchronous. by_kernel: src is known to be device memory that a kernel may read, so a short read
+  // may take launch_read_words.
+  void d2h(void* dst, const void* src, size_t bytes, bool by_kernel = true);
+  // Coherent pinned host memory that small gathers write directly from the device (zero copy),
+  // and behind it the flag that takes a gather's call number when its words are there.
   uint32_t* gather_host = nullptr;
   uint32_t* gather_host_dev = nullptr;  // the device's address of the same memory
   static constexpr size_t gather_host_words = 16384;
+  uint32_t gather_call = 0;
+  uint32_t* gather_flag() const { return gather_host_dev + gather_host_words; }
+  // Waits for gather number gather_call, the last work put on the main stream: polls its flag, and
+  // after GATHER_POLL_US (work queued before it still runs, or the device has failed) synchronises.
+  // The runtime retires finished launches only when the stream is synchronised, so every
+  // GATHER_POLLS-th wait does that in any case.
+  // Read-backs of up to this many words go the same way: against the copy engine and a synchronise, 8.0
+  // and 12.9 us for 8 words, 10.7 and 13.0 for 4096, 13.3 and 10.0 for 8192 (one workgroup's stores).
+  static constexpr size_t READ_WORDS = 4096;
+  static constexpr long GATHER_POLL_US = 500;
+  static constexpr uint32_t GATHER_POLLS = 32;
+  uint32_t polls = 0;
+  void wait_gather();
   uint8_t* d2h_pinned = nullptr;  // read-backs of up to d2h_cap bytes land here first
   static constexpr size_t d2h_cap = 4u << 20;
   // Pinned host memory for asynchronous read-backs on the main stream (kept and grown as needed;
