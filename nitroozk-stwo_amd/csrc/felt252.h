@@ -4,11 +4,9 @@
 // which calls starknet-crypto's poseidon_hash, poseidon_hash_many and poseidon_permute_comp.
 //
 // An element enters and leaves as eight little-endian 32-bit limbs (F), canonical. Inside the
-// permutation it is in Montgomery form (M): nine limbs of 29 bits in 32-bit registers, R = 2^261.
-// Radix 2^29 leaves room in each limb: a product column (at most 9 products of limbs below 2^30)
-// accumulates in one 64-bit register with no carry handling, and sums are limb-wise additions whose
-// carries are propagated once. p = 1 (mod 2^29), so the Montgomery factor of each column is minus
-// its low limb, and p's limbs are zero except limb 0 (1), limb 6 (17 2^18) and limb 8 (2^19).
+// permutation it is in Montgomery form (M): nine signed limbs of 29 bits in 32-bit registers, R =
+// 2^261. Radix 2^29 leaves room in each limb: a product column accumulates in one 64-bit register with
+// no carry handling, and sums are limb-wise additions whose carries move once, all limbs at a time.
 //
 // The permutation (state of 3): 4 full rounds (add 3 constants, cube all three), 83 partial rounds
 // (add one constant to the last element, cube it), 4 full rounds; each round ends with the MDS mix
@@ -200,87 +198,158 @@ constexpr F RC_NORMAL[107] = {
     {{0xdc5717a5u, 0xbf1d9ac2u, 0xabd8af54u, 0x7606836eu, 0xa13b7f2cu, 0xf180b1a8u, 0x92db5099u, 0x051274d0u}},
     {{0xbfff0c5bu, 0x861a8db0u, 0x0d9cdbedu, 0xf415e14fu, 0xaa4ca528u, 0x7ad0fb7au, 0xb8eb75e1u, 0x061fc552u}},
 };
-// ---- Montgomery form in radix 2^29 -----------------------------------------------------------
+// ---- Montgomery form in radix 2^29, signed limbs ---------------------------------------------
+// p = 1 + 17 2^192 + 2^251: its limb 0 is 1, limb 6 is 17 2^18, limb 8 is 2^19. Normalized means limbs 0-7
+// within 2^28 + 4 of zero; a limb of a sum of such may reach 7.5 2^28.
 constexpr uint32_t MASK29 = (1u << 29) - 1;
+constexpr int32_t HALF29 = 1 << 28, P6 = 17 << 18, P8 = 1 << 19;
 struct M {
-  uint32_t w[9];
+  int32_t w[9];
 };
 
-// F (any value below 2^256) -> nine 29-bit limbs
+// F (any value below 2^256) -> nine 29-bit limbs, none negative
 SHD constexpr M to_radix29(const F& a) {
   M r{};
   for (int i = 0; i < 9; ++i) {
     const int bit = 29 * i, w = bit / 32, sh = bit % 32;
     uint64_t v = a.w[w];
     if (w + 1 < 8) v |= (uint64_t)a.w[w + 1] << 32;
-    r.w[i] = (uint32_t)(v >> sh) & MASK29;
+    r.w[i] = (int32_t)((uint32_t)(v >> sh) & MASK29);
   }
   return r;
 }
-// nine 29-bit limbs of a value below 2^256 -> F
+// the value of the limbs, at least 0 and below 2^256 -> F
 SHD constexpr F from_radix29(const M& a) {
   F r = zero();
+  int32_t c = 0;
   for (int i = 0; i < 9; ++i) {
     const int bit = 29 * i, w = bit / 32, sh = bit % 32;
-    const uint64_t v = (uint64_t)a.w[i] << sh;
+    const int32_t x = a.w[i] + c;
+    c = x >> 29;
+    const uint64_t v = (uint64_t)(i < 8 ? (uint32_t)x & MASK29 : (uint32_t)x) << sh;
     r.w[w] |= (uint32_t)v;
     if (w + 1 < 8) r.w[w + 1] |= (uint32_t)(v >> 32);
   }
   return r;
 }
 
-// a b 2^-261 (mod p) by product scanning: column k gathers a_i b_j (i + j = k) and the reduction
-// terms m_i p_j in 64-bit accumulators; for k < 9 the factor m_k = -acc (mod 2^29) clears the
-// column (p's limb 0 is 1: acc + m_k is a multiple of 2^29, and its quotient is the carry out),
-// above that the columns are the result's limbs. Inputs: limbs below 2^30 (a column then stays
-// below 2^64); output: limbs 0-7 below 2^29, value below a b / 2^261 + p (below 2 p for inputs
-// below 32 p).
+// Constants that the device takes from registers: as literals, the compiler would turn these
+// multiply-adds into shifts and 64-bit additions, twice the instructions.
+struct MulConst {
+  int32_t one, p6, p8;
+  int64_t start[4];  // of columns 0-5, 6-7, 8-14, 15-16
+};
+constexpr MulConst MUL_CONST = {1, -P6, -P8, {HALF29, (int64_t)HALF29 * (1 + P6), (int64_t)HALF29 * (1 + P6 + P8),
+                                             (int64_t)HALF29 * (1 + P8)}};
+__device__ inline MulConst mul_const_device() {
+  MulConst k = MUL_CONST;
+  asm("" : "+s"(k.one), "+s"(k.p6), "+s"(k.p8));
+  asm("" : "+s"(k.start[0]), "+s"(k.start[1]), "+s"(k.start[2]), "+s"(k.start[3]));
+  return k;
+}
+SHD constexpr MulConst mul_const() {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (!__builtin_is_constant_evaluated()) return mul_const_device();
+#endif
+  return MUL_CONST;
+}
+
+// a b 2^-261 (mod p) by product scanning: column k gathers a_i b_j (i + j = k) in a signed 64-bit
+// accumulator. p's limb 0 being 1, the factor that clears column k < 9 is minus its signed low 29 bits
+// c, which adds -c 17 2^18 to column k + 6 and -c 2^19 to column k + 8. Every column starts at 2^28, so
+// that a mask and a shift split off c + 2^28 and the carry; later columns start at what the 2^28 in the
+// factors' place adds too much. Two instructions of masks and shifts a column besides the multiply-adds
+// (carries are added by one as well): 157 in all, 129 for a square, against some 175 and no square
+// on unsigned limbs. Inputs: normalized; accumulators
+// stay below 2^59.4. Output: normalized, within 0.51 p of zero for inputs within 2^7 p.
+template <bool SQUARE>
 SHD constexpr M mul29(const M& a, const M& b) {
-  uint32_t m[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const MulConst q = mul_const();
+  int32_t twice[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, lo[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if (SQUARE)
+    for (int i = 0; i < 9; ++i) twice[i] = a.w[i] + a.w[i];
   M r{};
-  uint64_t acc = 0;
+  int32_t carry = 0;
 #pragma unroll
   for (int k = 0; k < 17; ++k) {
-    // two partial sums per column (products of even and odd i, the even one starting from the
-    // carry in): chains of multiply-adds of which only one waits for the previous column
-    uint64_t e = acc, o = 0;
+    int64_t acc = q.start[k < 6 ? 0 : k < 8 ? 1 : k < 15 ? 2 : 3];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
       const int j = k - i;
-      if (j >= 0 && j < 9) {
-        if (i & 1)
-          o += (uint64_t)a.w[i] * b.w[j];
-        else
-          e += (uint64_t)a.w[i] * b.w[j];
-      }
+      if (j < 0 || j > 8) continue;
+      if (!SQUARE)
+        acc += (int64_t)a.w[i] * b.w[j];
+      else if (i <= j)
+        acc += (int64_t)(i < j ? twice[i] : a.w[i]) * a.w[j];
     }
-    if (k >= 6 && k - 6 < 9) o += (uint64_t)m[k - 6] * (17u << 18);
-    if (k >= 8 && k - 8 < 9) e += (uint64_t)m[k - 8] << 19;
-    acc = e + o;
-    if (k < 9) {
-      m[k] = (0u - (uint32_t)acc) & MASK29;
-      acc = (acc + m[k]) >> 29;
-    } else {
-      r.w[k - 9] = (uint32_t)acc & MASK29;
-      acc >>= 29;
-    }
+    if (k) acc += (int64_t)carry * q.one;
+    if (k >= 6 && k < 15) acc += (int64_t)lo[k - 6] * q.p6;
+    if (k >= 8) acc += (int64_t)lo[k - 8] * q.p8;
+    const int32_t l = (int32_t)((uint32_t)acc & MASK29);
+    if (k < 9)
+      lo[k] = l;
+    else
+      r.w[k - 9] = l - HALF29;
+    carry = (int32_t)(acc >> 29);
   }
-  r.w[8] = (uint32_t)acc;
+  r.w[8] = carry;
+  return r;
+}
+SHD constexpr M mul(const M& a, const M& b) { return mul29<false>(a, b); }
+SHD constexpr M square(const M& a) { return mul29<true>(a, a); }
+
+// Carries, each by one limb: limbs 0-7 normalized for limbs within 7 2^28 of zero, limb 8 whole.
+SHD constexpr M carry(const M& x) {
+  M r{};
+  int32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int32_t v = x.w[i] + HALF29;
+    r.w[i] = (int32_t)((uint32_t)v & MASK29) - HALF29 + c;
+    c = v >> 29;
+  }
+  r.w[8] = x.w[8] + c;
+  return r;
+}
+// x less the multiple of p that leaves the top limb within 2^18 of zero before the carries (within
+// 2^250 + 2^235 of zero then); limbs within 7.5 2^28 of zero, values within 2^5 p.
+SHD M reduce_top(const M& x) {
+  const int32_t h = (x.w[8] + (1 << 18)) >> 19;
+  M y = x, r{};
+  y.w[0] -= h;
+  y.w[6] -= 17 * h * (1 << 18);
+  y.w[8] -= h * P8;
+  int32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    // (w + 2^28) >> 29, which could overflow; that times 2^29 less w is minus a normalized limb
+    const int32_t v = ((y.w[i] >> 28) + 1) >> 1;
+    r.w[i] = (int32_t)((uint32_t)y.w[i] - ((uint32_t)v << 29)) + c;
+    c = v;
+  }
+  r.w[8] = y.w[8] + c;
   return r;
 }
 
-constexpr M R2M = to_radix29(pow2_mod_p(522));  // R^2 mod p
-// canonical F -> Montgomery form (below 1.04 p)
-SHD constexpr M to_mont(const F& a) { return mul29(to_radix29(a), R2M); }
-// Montgomery form (limbs below 2^29, value below 2^261) -> canonical F
+constexpr M R2M = carry(to_radix29(pow2_mod_p(522)));  // R^2 mod p
+// canonical F (any value below 2^256, in fact) -> Montgomery form
+SHD constexpr M to_mont(const F& a) { return mul(carry(to_radix29(a)), R2M); }
+// Montgomery form (limbs within 7 2^28 of zero) -> canonical F
 SHD constexpr F from_mont(const M& a) {
-  const F r = from_radix29(mul29(a, M{{1, 0, 0, 0, 0, 0, 0, 0, 0}}));  // at most p
+  M y = mul(carry(a), M{{1, 0, 0, 0, 0, 0, 0, 0, 0}});  // above -p
+  y.w[0] += 1;
+  y.w[6] += P6;
+  y.w[8] += P8;
+  const F r = from_radix29(y);
   return geq_p(r) ? sub_p(r) : r;
 }
 
 constexpr M ONE = to_mont(from_u64(1));
 constexpr M TWO = to_mont(from_u64(2));
 constexpr M THREE = to_mont(from_u64(3));
+// 1/2, which is (p + 1) / 2, and 1/4
+constexpr M HALF = to_mont(F{{1, 0, 0, 0, 0, 0x80000000u, 8, 0x04000000u}});
+constexpr M QUARTER = mul(HALF, HALF);
 
 struct RoundConstants {
   M c[107];
@@ -293,144 +362,79 @@ constexpr RoundConstants make_round_constants() {
 constexpr RoundConstants RC = make_round_constants();
 
 // ---- the permutation's arithmetic: reduced lazily, no branches ----------------------------------
-// limb-wise sum
-SHD M addl(const M& a, const M& b) {
-  M r;
+// x f + y g limb by limb
+SHD constexpr M lin(const M& x, int32_t f, const M& y, int32_t g) {
+  M r{};
 #pragma unroll
-  for (int i = 0; i < 9; ++i) r.w[i] = a.w[i] + b.w[i];
+  for (int i = 0; i < 9; ++i) r.w[i] = f * x.w[i] + g * y.w[i];
   return r;
 }
-// carries of limbs below 2^32 - 8: limbs 0-7 below 2^29 after it
-SHD M carry(const M& x) {
-  M r;
-  uint32_t c = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t v = x.w[i] + c;
-    r.w[i] = v & MASK29;
-    c = v >> 29;
-  }
-  r.w[8] = x.w[8] + c;
-  return r;
-}
-// x - (q - 1) p for q = floor(x / 2^251) >= 1 (x itself for q = 0): congruent to x and below
-// 2^251 + p < 2 p, for x with normalized limbs and q at most 120 (a value below 2^257.9: the limb-6
-// term 17 2^18 (q - 1) stays below 2^29). (q - 1) p touches limbs 0, 6 and 8 only; the borrows are
-// -1 or 0.
-SHD M reduce_top(const M& x) {
-  const uint32_t q = x.w[8] >> 19;
-  const uint32_t k = q - (q != 0u ? 1u : 0u);
-  const uint32_t sub[9] = {k, 0u, 0u, 0u, 0u, 0u, (17u << 18) * k, 0u, k << 19};
-  M r;
-  int32_t c = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int32_t v = (int32_t)x.w[i] - (int32_t)sub[i] + c;
-    r.w[i] = (uint32_t)v & MASK29;
-    c = v >> 29;  // arithmetic: -1 or 0
-  }
-  r.w[8] = (uint32_t)((int32_t)x.w[8] - (int32_t)sub[8] + c);
-  return r;
-}
-// The value v plus a multiple of 2^29 moved down from each limb to the one below: the same value
-// with limbs 0-7 at least D (2^29 - 1), so that subtracting D times a normalized element limb by
-// limb leaves every limb non-negative.
-constexpr M borrowed(const M& v, uint32_t D) {
-  M r = v;
-  for (int i = 0; i < 8; ++i) {
-    r.w[i] += D << 29;
-    r.w[i + 1] -= D;
-  }
-  return r;
-}
-constexpr M from_small_multiple_of_p(uint32_t k) {  // k p in radix 2^29, k < 32
-  return M{{k, 0u, 0u, 0u, 0u, 0u, (17u << 18) * k, 0u, k << 19}};
-}
-// 5 p and 7 p, borrowed for subtracting 2 s1 and 3 s2 (their top limbs 5 2^19 and 7 2^19 exceed
-// 2 and 3 times the top limb of elements below 2.01 p, plus the borrow); 21 p for 2 s1 with s1
-// below 10.3 p (the partial rounds that follow a round without reduction)
-constexpr M K5P = borrowed(from_small_multiple_of_p(5), 2);
-constexpr M K7P = borrowed(from_small_multiple_of_p(7), 3);
-constexpr M K21P = borrowed(from_small_multiple_of_p(21), 2);
-
-// t = s0 + s1 + s2 -> (t + 2 s0, t - 2 s1, t - 3 s2) for normalized inputs below 2.01 p. The
-// unnormalized outputs stay below 9.1 p, 10.1 p and 12.1 p (limbs below 7 2^29); the first two are
-// brought below 2.01 p, the third (which is cubed next) only normalized.
-SHD void mix(M* s) {
-  M a, b, c;
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    const uint32_t t = s[0].w[i] + s[1].w[i] + s[2].w[i];
-    a.w[i] = t + 2u * s[0].w[i];
-    b.w[i] = t + K5P.w[i] - 2u * s[1].w[i];
-    c.w[i] = t + K7P.w[i] - 3u * s[2].w[i];
-  }
-  s[0] = reduce_top(carry(a));
-  s[1] = reduce_top(carry(b));
-  s[2] = carry(c);
-}
-// The partial rounds' mix, reducing s0 and s1 every other round (s2, cubed next, is only
-// normalized). REDUCE = false takes s0, s1 below 2.01 p and leaves them normalized below 9.3 p and
-// 10.3 p (c below 12.3 p); REDUCE = true takes those, subtracts 2 s1 from 21 p, and brings a (below
-// 39.2 p) and b (below 41.7 p) below 2 p (c below 27.7 p, its cube below 1.06 p). Limbs stay below
-// 2^32 - 8 either way: every input is normalized.
-template <bool REDUCE>
-SHD void mix_partial(M* s) {
-  M a, b, c;
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    const uint32_t t = s[0].w[i] + s[1].w[i] + s[2].w[i];
-    a.w[i] = t + 2u * s[0].w[i];
-    b.w[i] = t + (REDUCE ? K21P.w[i] : K5P.w[i]) - 2u * s[1].w[i];
-    c.w[i] = t + K7P.w[i] - 3u * s[2].w[i];
-  }
-  if (REDUCE) {
-    s[0] = reduce_top(carry(a));
-    s[1] = reduce_top(carry(b));
-  } else {
-    s[0] = carry(a);
-    s[1] = carry(b);
-  }
-  s[2] = carry(c);
-}
-SHD M cube(const M& x) { return mul29(mul29(x, x), x); }
-// each element plus its constant (limbs below 2^30, value below 14 p) cubed: below 1.2 p
+SHD constexpr M addl(const M& a, const M& b) { return lin(a, 1, b, 1); }
+SHD M cube(const M& x) { return mul(square(x), x); }
+// Each element plus its constant cubed, then t = s0 + s1 + s2 -> (t + 2 s0, t - 2 s1, t - 3 s2). Elements
+// come and go unnormalized: limbs within 5, 3 and 4 2^28 of zero, values within 2.6 p.
 SHD void full_round(M* s, int k) {
-  for (int i = 0; i < 3; ++i) s[i] = cube(addl(s[i], RC.c[k + i]));
-  mix(s);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) s[i] = cube(carry(addl(s[i], RC.c[k + i])));
+  M a, b, c;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const int32_t u = s[0].w[i] + s[1].w[i], d = s[0].w[i] - s[1].w[i];
+    a.w[i] = u + s[2].w[i] + 2 * s[0].w[i];
+    b.w[i] = d + s[2].w[i];
+    c.w[i] = u - 2 * s[2].w[i];
+  }
+  s[0] = a;
+  s[1] = b;
+  s[2] = c;
 }
-// poseidon_permute_comp on a Montgomery-form state: elements with limbs below 2^30 and values
-// below 3.1 p (Montgomery forms of canonical values, or a permutation's outputs plus an absorbed
-// value). Outputs: s0 and s1 below 2.01 p, s2 below 12.1 p, all normalized (from_mont reduces
-// fully). The 83 partial rounds run as 41 pairs (without, then with the reduction of s0 and s1)
-// and one round without it, whose outputs (below 12.3 p plus a constant: under the full rounds'
-// 14 p) go to the last full rounds. One copy of the code per program: the device calls it, it is
-// not inlined.
+// poseidon_permute_comp on a Montgomery-form state, limbs within 6 2^28 of zero and values within 6 p;
+// the outputs are full_round's.
+//
+// In the partial rounds only x_n = (s2_n + constant)^3 is not linear: with 2 w_n = s0_n + s1_n the mix
+// says w_{n+1} = 2 w_n + 4 w_{n-1} + x_n and s2_{n+1} = 2 (w_n - x_n), which takes one reduction a round
+// in place of s0's and s1's. It starts from 4 w_{-1} = s0 - s1 and ends in s0 = w + 2 w_prev,
+// s1 = w - 2 w_prev. With the signed products, 475 instructions a partial round: a layer of 2^17 nodes 218 ->
+// 187 us (two waves a SIMD), of 2^14 115 -> 99 us (one wave, the chain's latency). w is kept within 2^250 + 2^235 of zero: the sum's limbs stay within 7.01 2^28.
+// One copy of the code per program: the device calls it, it is not inlined.
 __host__ __device__ __attribute__((noinline)) inline void permute(M* s) {
   for (int i = 0; i < 3; ++i) s[i] = carry(s[i]);
   int k = 0;
-  for (int r = 0; r < 4; ++r, k += 3) full_round(s, k);
 #ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll 1
 #endif
-  for (int r = 0; r < 41; ++r, k += 2) {
-    s[2] = cube(addl(s[2], RC.c[k]));
-    mix_partial<false>(s);
-    s[2] = cube(addl(s[2], RC.c[k + 1]));
-    mix_partial<true>(s);
+  for (int r = 0; r < 4; ++r, k += 3) full_round(s, k);
+  const M s0 = carry(s[0]), s1 = carry(s[1]);
+  M w = mul(carry(addl(s0, s1)), HALF), prev = mul(carry(lin(s0, 1, s1, -1)), QUARTER), s2 = s[2];
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll 1
+#endif
+  for (int r = 0; r < 83; ++r, ++k) {
+    const M x = cube(carry(addl(s2, RC.c[k])));
+    M next;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      s2.w[i] = 2 * (w.w[i] - x.w[i]);
+      next.w[i] = 2 * (2 * prev.w[i] + w.w[i]) + x.w[i];
+    }
+    prev = w;
+    w = reduce_top(next);
   }
-  s[2] = cube(addl(s[2], RC.c[k]));
-  mix_partial<false>(s);
-  ++k;
+  s[2] = s2;
+  s[0] = lin(w, 1, prev, 2);
+  s[1] = lin(w, 1, prev, -2);
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll 1
+#endif
   for (int r = 0; r < 4; ++r, k += 3) full_round(s, k);
 }
-// poseidon_hash(x, y) (Montgomery form in and out)
+// poseidon_hash(x, y) (Montgomery form in and out; in as permute takes it)
 SHD M hash2(const M& x, const M& y) {
   M s[3] = {x, y, TWO};
   permute(s);
   return s[0];
 }
-// poseidon_hash_many, absorbing one value at a time (Montgomery form; absorbed values below 1.1 p)
+// poseidon_hash_many, absorbing one value at a time (Montgomery form, normalized)
 struct Sponge {
   M s[3] = {M{}, M{}, M{}};
   M pending = M{};

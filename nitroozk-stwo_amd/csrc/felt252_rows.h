@@ -10,37 +10,33 @@
 // elsewhere (17 2^18 six columns up, 2^19 eight columns up) comes in two steps, first for columns 0..5,
 // then for 6..8, which depend on them. Carries move by one lane, all lanes at once, between the steps:
 // every value fits 32 bits after one of them. Products lie in (-p, p); a product is 65 instructions (57
-// when the shifted operand is at hand) against 260 for one lane.
+// when the shifted operand is at hand) against 157 for one lane.
 //
-// The mix works limb by limb in every lane. s0 and s1 are brought near zero after every round: the top
-// limb's multiple of 2^251 is taken off with a multiple of p, then the carries move once; s2 is normalized
-// with its next constant. Ranges, checked over extreme limbs and whole permutations: accumulators below
-// 2^59.1 (hi words of the first carry below 2^31), sums of the mix below 2^30.4, values below 4 p.
+// Sums work limb by limb in every lane; carries move once before a product, and the partial rounds'
+// recurrence (felt252.h) reduces one value a round. Ranges, checked over extreme limbs and whole
+// permutations: accumulators below 2^59.4 (hi words of the first carry below 2^31), sums within 7.1 2^28.
 #pragma once
 #include "felt252.h"
 
 namespace sh {
 namespace f252 {
 
-// Per lane of a row: the round constants, then R^2, the Montgomery forms of 1 and 2, and 1, all with
-// balanced limbs.
-constexpr int ROWS_R2 = 107, ROWS_ONE = 108, ROWS_TWO = 109, ROWS_UNIT = 110, ROWS_N = 111;
+// Per lane of a row: the round constants, then R^2, the Montgomery forms of 1 and 2, 1, and the Montgomery
+// forms of 1/2 and 1/4.
+constexpr int ROWS_R2 = 107, ROWS_ONE = 108, ROWS_TWO = 109, ROWS_UNIT = 110,
+              ROWS_HALF = 111, ROWS_QUARTER = 112, ROWS_N = 113;
 struct RowTable { int32_t v[ROWS_N * 16]; };
-constexpr void balance_into(int32_t* out, const M& m) {
-  int32_t c = 0;
-  for (int i = 0; i < 8; ++i) {
-    const int32_t x = (int32_t)m.w[i] + c;
-    c = x >= (1 << 28) ? 1 : 0;
-    out[i] = x - (c << 29);
-  }
-  out[8] = (int32_t)m.w[8] + c;
+constexpr void row_into(RowTable& t, int row, const M& m) {
+  for (int i = 0; i < 9; ++i) t.v[16 * row + i] = m.w[i];
 }
 constexpr RowTable make_row_table() {
   RowTable t{};
-  for (int i = 0; i < 107; ++i) balance_into(t.v + 16 * i, RC.c[i]);
-  balance_into(t.v + 16 * ROWS_R2, R2M);
-  balance_into(t.v + 16 * ROWS_ONE, ONE);
-  balance_into(t.v + 16 * ROWS_TWO, TWO);
+  for (int i = 0; i < 107; ++i) row_into(t, i, RC.c[i]);
+  row_into(t, ROWS_R2, R2M);
+  row_into(t, ROWS_ONE, ONE);
+  row_into(t, ROWS_TWO, TWO);
+  row_into(t, ROWS_HALF, HALF);
+  row_into(t, ROWS_QUARTER, QUARTER);
   t.v[16 * ROWS_UNIT] = 1;
   return t;
 }
@@ -87,15 +83,18 @@ struct Row {
   }
   __device__ __forceinline__ int32_t at(int row) const { return tab[16 * row]; }
 
-  // Carries of 32-bit limbs (sums below 2^31), by one lane; the top limb keeps everything.
+  // Carries, by one lane, of limbs within 7 2^28 of zero; the top limb keeps everything.
   __device__ __forceinline__ int32_t carry(int32_t x) const {
     const int32_t lo = __builtin_amdgcn_sbfe(x, 0, width), hi = (x + round_up) >> width;
     return lo + row_up<1>(hi);
   }
-  // Minus the multiple of p that the top limb's multiple of 2^251 calls for, then the carries.
-  __device__ __forceinline__ int32_t normalize(int32_t x) const {
+  // reduce_top: minus the multiple of p that leaves the top limb near zero, then the carries, of limbs
+  // within 7.5 2^28 of zero (the rounded shift in two steps, as adding half could overflow).
+  __device__ __forceinline__ int32_t reduce(int32_t x) const {
     const int32_t h = row_bcast<8>((x + (1 << 18)) >> 19);
-    return carry(x + __mul24(h, minus_p));
+    const int32_t y = x + __mul24(h, minus_p);
+    const int32_t lo = __builtin_amdgcn_sbfe(y, 0, width), hi = ((y >> (width - 1)) + 1) >> 1;
+    return lo + row_up<1>(hi);
   }
 
   struct Shifted { int32_t s[9], top; };  // b moved up by 0..8 lanes, and its top limb in every lane
@@ -138,37 +137,37 @@ struct Row {
     const Shifted s = shifts(x);
     return mul(mul(x, s), s);
   }
-  __device__ __forceinline__ void mix(int32_t* s) const {
-    const int32_t u = s[0] + s[2], w = s[0] + s[1];
-    const int32_t a = u + s[1] + 2 * s[0], b = u - s[1], c = w - 2 * s[2];
-    s[0] = normalize(a);
-    s[1] = normalize(b);
-    s[2] = c;
-  }
   __device__ __forceinline__ void full_rounds(int32_t* s, int r) const {
 #pragma unroll 1
     for (int i = 0; i < 4; ++i, r += 3) {
 #pragma unroll
       for (int j = 0; j < 3; ++j) s[j] = cube(carry(s[j] + at(r + j)));
-      mix(s);
+      const int32_t u = s[0] + s[1], d = s[0] - s[1];
+      s[0] = u + s[2] + 2 * s[0];
+      s[1] = d + s[2];
+      s[2] = u - 2 * s[2];
     }
   }
-  // poseidon_permute_comp: s0 and s1 normalized in and out (s2 below 2^30.4 in every limb).
+  // poseidon_permute_comp, as permute() in felt252.h.
   __device__ __forceinline__ void permute(int32_t* s) const {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s[j] = carry(s[j]);
     full_rounds(s, 0);
-    // s0 and s1 wait unnormalized for the next round, whose product has idle slots for that
-    int32_t rc = at(12), a = s[0], b = s[1];
+    const int32_t s0 = carry(s[0]), s1 = carry(s[1]);
+    int32_t w = mul(carry(s0 + s1), shifts(at(ROWS_HALF))), prev = mul(carry(s0 - s1), shifts(at(ROWS_QUARTER)));
+    // w_{n+1} waits unreduced for the next round, whose product has idle slots for that
+    int32_t rc = at(12);
 #pragma unroll 1
     for (int r = 12; r < 95; ++r) {
-      const int32_t next = at(r + 1), s0 = normalize(a), s1 = normalize(b), u = s0 + s1;
-      const int32_t x = cube(carry(s[2] + rc));
-      a = u + 2 * s0 + x;
-      b = s0 - s1 + x;
-      s[2] = u - 2 * x;
+      const int32_t next = at(r + 1), cur = reduce(w), x = cube(carry(s[2] + rc));
+      s[2] = 2 * (cur - x);
+      w = 2 * (2 * prev + cur) + x;
+      prev = cur;
       rc = next;
     }
-    s[0] = normalize(a);
-    s[1] = normalize(b);
+    const int32_t last = reduce(w);
+    s[0] = last + 2 * prev;
+    s[1] = last - 2 * prev;
     full_rounds(s, 95);
   }
   // Limb k of eight words in memory, and of eight words that every lane of the row holds; Montgomery form.
@@ -182,22 +181,14 @@ struct Row {
     const M m = to_radix29(f);
     uint32_t v = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < 9; ++j) v = k == j ? m.w[j] : v;
+    for (uint32_t j = 0; j < 9; ++j) v = k == j ? (uint32_t)m.w[j] : v;
     return (int32_t)v;
   }
   // The canonical value of a state element, in every lane of the row.
   __device__ __forceinline__ F from_mont(int32_t x) const {
-    const int32_t y = mul(x, shifts(at(ROWS_UNIT)));  // in (-p, p): p is added, which makes it positive
-    const int32_t l[9] = {row_bcast<0>(y), row_bcast<1>(y), row_bcast<2>(y), row_bcast<3>(y), row_bcast<4>(y),
-                          row_bcast<5>(y), row_bcast<6>(y), row_bcast<7>(y), row_bcast<8>(y)};
-    M m;
-    int32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      const int32_t v = l[i] + (i == 0 ? 1 : i == 6 ? 17 << 18 : i == 8 ? 1 << 19 : 0) + c;
-      m.w[i] = i < 8 ? (uint32_t)v & MASK29 : (uint32_t)v;
-      c = v >> 29;
-    }
+    const int32_t y = mul(carry(x), shifts(at(ROWS_UNIT))) - minus_p;  // above -p before p is added
+    const M m{{row_bcast<0>(y), row_bcast<1>(y), row_bcast<2>(y), row_bcast<3>(y), row_bcast<4>(y), row_bcast<5>(y),
+               row_bcast<6>(y), row_bcast<7>(y), row_bcast<8>(y)}};
     const F r = from_radix29(m);
     return geq_p(r) ? sub_p(r) : r;
   }
