@@ -11,11 +11,11 @@
 // roots and runs the channel step. Layers of at most 2^8 values run in one workgroup, all of them
 // in one launch (fri_small_kernel), with each layer's values kept in LDS for the next fold.
 //
-// Inside a workgroup a Merkle level is held in LDS word-major (word k of node i at k * n + i), so a
-// lane reads both children's word k with one 8-byte load and a wave's loads hit distinct banks.
-// Wide levels hash one node per lane (Blake2s is issue-bound: one wave per SIMD already reaches
-// peak throughput); levels of at most 64 parents hash one node per quad of lanes, which has about
-// half the latency of one lane.
+// Inside a workgroup a wide Merkle level is held in LDS word-major (word k of node i at k * n + i), so a
+// lane reads both children's word k with one 8-byte load and a wave's loads hit distinct banks; it
+// hashes one node per lane (Blake2s is issue-bound: one wave per SIMD already reaches peak throughput).
+// Levels of at most 64 parents hash one node per quad of lanes, which has a third of the latency of one
+// lane, from nodes held as the quads' messages (blake2s_compress_quad_lds).
 #include <stdexcept>
 #include <type_traits>
 #include "blake2s.h"
@@ -90,125 +90,130 @@ __device__ __forceinline__ void leaf_hash(qm31 v, uint32_t h[8]) {
   blake2s_compress(h, m, 16, true);
 }
 
-// The m parents of the 2m nodes in `in` (word k of node i at in[k * 2m + i]) into `out` (word k of
-// parent p at out[k * m + p]), each parent also stored as 8 consecutive words at g + 8 p. Called by
-// every thread of the workgroup; ends with a barrier.
-__device__ __forceinline__ void fl_level(const uint32_t* in, uint32_t* out, uint32_t m, uint32_t* __restrict__ g) {
-  const uint32_t t = threadIdx.x, si = 2 * m;
-  if (m > 64) {
-    for (uint32_t p = t; p < m; p += FL_THREADS) {
-      uint32_t msg[16], h[8];
+constexpr uint32_t FL_QUADS = 64;  // parents of the widest level hashed by quads
+struct QuadBufs {
+  uint32_t a[FL_QUADS * QUAD_MSG], b[FL_QUADS / 2 * QUAD_MSG + 1];
+};
+
+// Node i of n in a workgroup's level: word-major in `wide`, or (levels that quads hash) a half message.
+__device__ __forceinline__ void fl_put(uint32_t* wide, QuadBufs& quads, uint32_t n, uint32_t i, const uint32_t h[8]) {
+  if (n > 2 * FL_QUADS) {
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint2 w = *reinterpret_cast<const uint2*>(in + k * si + 2 * p);
-        msg[k] = w.x;
-        msg[8 + k] = w.y;
-      }
-      blake2s_init(h);
-      blake2s_compress(h, msg, 64, true);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) out[k * m + p] = h[k];
-      store8(g + 8 * p, h);
-    }
+    for (int k = 0; k < 8; ++k) wide[k * n + i] = h[k];
   } else {
-    const uint32_t p = t >> 2, q = t & 3;
-    if (p < m) {  // whole quads are active or not
-      uint32_t msg[16];
+    const uint32_t o = quad_node(i);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint2 w = *reinterpret_cast<const uint2*>(in + k * si + 2 * p);
-        msg[k] = w.x;
-        msg[8 + k] = w.y;
-      }
-      uint32_t hA, hB;
-      blake2s_init_quad(q, hA, hB);
-      blake2s_compress_quad(hA, hB, msg, 64, true, q);
-      out[q * m + p] = hA;
-      out[(4 + q) * m + p] = hB;
-      gmem(g)[8 * p + q] = hA;
-      gmem(g)[8 * p + 4 + q] = hB;
+    for (int k = 0; k < 8; ++k) quads.a[o + k] = h[k];
+  }
+}
+
+// The m > 64 parents of the 2m nodes in `in`, each parent also stored as 8 consecutive words at g + 8 p.
+// Called by every thread of the workgroup; ends with a barrier.
+__device__ __forceinline__ void fl_wide_level(const uint32_t* in, uint32_t* out, QuadBufs& quads, uint32_t m,
+                                              uint32_t* __restrict__ g) {
+  const uint32_t si = 2 * m;
+  for (uint32_t p = threadIdx.x; p < m; p += FL_THREADS) {
+    uint32_t msg[16], h[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint2 w = *reinterpret_cast<const uint2*>(in + k * si + 2 * p);
+      msg[k] = w.x;
+      msg[8 + k] = w.y;
     }
+    blake2s_init(h);
+    blake2s_compress(h, msg, 64, true);
+    fl_put(out, quads, m, p, h);
+    store8(g + 8 * p, h);
+  }
+  __syncthreads();
+}
+// The m <= 64 parents of the messages in `in`, likewise.
+__device__ __forceinline__ void fl_quad_level(const uint32_t* in, uint32_t* out, const QuadSchedule& s, uint32_t m,
+                                              uint32_t* __restrict__ g) {
+  const uint32_t p = threadIdx.x >> 2, q = threadIdx.x & 3;
+  if (p < m) {  // whole quads are active or not
+    uint32_t hA, hB;
+    blake2s_init_quad(q, hA, hB);
+    blake2s_compress_quad_lds(hA, hB, in, s, 64, true, q);
+    const uint32_t o = quad_node(p);
+    out[o + q] = hA;
+    out[o + 4 + q] = hB;
+    gmem(g)[8 * p + q] = hA;
+    gmem(g)[8 * p + 4 + q] = hB;
   }
   __syncthreads();
 }
 
-// Hashes levels up from the n nodes held in `a` (word-major, row stride n) until one node remains,
-// alternating between the buffers a and b; `heap` is the layer's Merkle heap, `lev` the level of
-// the nodes in a and `first` the heap index of a's node 0 within that level. Returns the buffer
-// that holds the top node (row stride 1 at the end).
-__device__ __forceinline__ const uint32_t* fl_levels(uint32_t* a, uint32_t* b, uint32_t n, uint32_t lev, uint32_t first,
+// Hashes levels up from the n nodes held as fl_put left them (`a`: word-major) until one node remains;
+// `heap` is the layer's Merkle heap, `lev` the level of the nodes and `first` the heap index of node 0
+// within that level. Returns the top node's 8 words.
+__device__ __forceinline__ const uint32_t* fl_levels(uint32_t* a, uint32_t* b, QuadBufs& quads, const QuadSchedule& s,
+                                                     uint32_t n, uint32_t lev, uint32_t first,
                                                      uint32_t* __restrict__ heap) {
+  const auto up = [&] {
+    n >>= 1;
+    first >>= 1;
+    --lev;
+    return heap + 8 * (((size_t)1 << lev) - 1 + (size_t)first);
+  };
   uint32_t* in = a;
   uint32_t* out = b;
-  while (n > 1) {
-    const uint32_t m = n >> 1;
-    --lev;
-    fl_level(in, out, m, heap + 8 * (((size_t)1 << lev) - 1 + (size_t)(first >> 1)));
-    first >>= 1;
+  while (n > 2 * FL_QUADS) {
+    uint32_t* g = up();
+    fl_wide_level(in, out, quads, n, g);
     uint32_t* x = in;
     in = out;
     out = x;
-    n = m;
   }
-  return in;
+  while (n > 1) {  // the two buffers are named, so that their addresses are constants of the reads
+    uint32_t* g = up();
+    fl_quad_level(quads.a, quads.b, s, n, g);
+    if (n == 1) return quads.b;
+    g = up();
+    fl_quad_level(quads.b, quads.a, s, n, g);
+  }
+  return quads.a;
 }
 
-// The channel step on one quad of lanes (q = lane within the quad; all 4 active): st (digest and
-// n_draws, identical in the 4 lanes) absorbs the root and a QM31 is drawn, redrawing until all 8
-// drawn words are below 2P (draw_base_felts). On return st and alpha are identical in the 4 lanes;
-// alpha is P in every coordinate (not canonical) if 64 draws fail, which the host replay reports.
-__device__ __forceinline__ void fl_channel(uint32_t st[9], const uint32_t root[8], uint32_t q, uint32_t alpha[4]) {
-  uint32_t m[16];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) { m[k] = st[k]; m[8 + k] = root[k]; }
+// The channel step on the first quad of lanes (q = lane; all 4 active), whose schedule is s: the digest in
+// ch[0..7] absorbs the root and a QM31 is drawn, redrawing until all 8 drawn words are below 2P
+// (draw_base_felts). ch[0..8] is the new state (digest and n_draws) afterwards. Lane q writes words q and
+// q + 4 of the record (root, then alpha in words 8..11) and returns alpha's word q, which is P (not
+// canonical, which the host replay reports) if 64 draws fail.
+__device__ __forceinline__ uint32_t fl_channel(uint32_t* ch, const uint32_t* root, const QuadSchedule& s, uint32_t q,
+                                               uint32_t* __restrict__ rec) {
+  const uint32_t r_lo = root[q], r_hi = root[4 + q];
+  gmem(rec)[q] = r_lo;
+  gmem(rec)[4 + q] = r_hi;
+  ch[8 + q] = r_lo;
+  ch[12 + q] = r_hi;
+  quad_sync();
   uint32_t hA, hB;
   blake2s_init_quad(q, hA, hB);
-  blake2s_compress_quad(hA, hB, m, 64, true, q);
-  st[0] = quad_bcast<0>(hA); st[1] = quad_bcast<1>(hA); st[2] = quad_bcast<2>(hA); st[3] = quad_bcast<3>(hA);
-  st[4] = quad_bcast<0>(hB); st[5] = quad_bcast<1>(hB); st[6] = quad_bcast<2>(hB); st[7] = quad_bcast<3>(hB);
-  st[8] = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) alpha[k] = P;
-  for (int attempt = 0; attempt < 64; ++attempt) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) m[k] = st[k];
-    m[8] = st[8];  // n_draws, little endian, then the zero byte and zero padding
-#pragma unroll
-    for (int k = 9; k < 16; ++k) m[k] = 0;
-    st[8] += 1;
+  blake2s_compress_quad_lds(hA, hB, ch, s, 64, true, q);
+  quad_sync();
+  ch[q] = hA;
+  ch[4 + q] = hB;
+  ch[8 + q] = 0;  // n_draws, little endian, then the zero byte and zero padding
+  ch[12 + q] = 0;
+  uint32_t alpha = P;
+  for (uint32_t attempt = 0; attempt < 64; ++attempt) {
+    if (q == 0) ch[8] = attempt;
+    quad_sync();
     blake2s_init_quad(q, hA, hB);
-    blake2s_compress_quad(hA, hB, m, 37, true, q);
+    blake2s_compress_quad_lds(hA, hB, ch, s, 37, true, q);
+    quad_sync();
+    if (q == 0) ch[8] = attempt + 1;
     uint32_t ok = (hA < 2 * P && hB < 2 * P) ? 1u : 0u;
     ok &= quad_perm<0x39>(ok);  // lanes (i, i + 1)
     ok &= quad_perm<0x4E>(ok);  // all four lanes
     if (ok) {
-      const uint32_t a = hA >= P ? hA - P : hA;  // lane k holds drawn word k
-      alpha[0] = quad_bcast<0>(a); alpha[1] = quad_bcast<1>(a); alpha[2] = quad_bcast<2>(a); alpha[3] = quad_bcast<3>(a);
+      alpha = hA >= P ? hA - P : hA;  // lane k holds drawn word k
       break;
     }
   }
-}
-
-// Lane q of the quad writes words q and q + 4 of the record (root, then alpha in words 8..11) and of
-// the channel state (n_draws from lane 0) to rec and st_out, and alpha word q to alpha_out when
-// given. Selects instead of indexing by q keep the arrays in registers.
-template <class StPtr, class AlphaPtr>
-__device__ __forceinline__ void fl_publish(uint32_t q, const uint32_t st[9], const uint32_t root[8],
-                                           const uint32_t alpha[4], uint32_t* __restrict__ rec, StPtr st_out,
-                                           AlphaPtr alpha_out) {
-  uint32_t r_lo = pin(root[0]), r_hi = pin(root[4]), a = pin(alpha[0]), s_lo = pin(st[0]), s_hi = pin(st[4]);
-#pragma unroll
-  for (uint32_t k = 1; k < 4; ++k) {
-    const uint32_t rl = pin(root[k]), rh = pin(root[4 + k]), ak = pin(alpha[k]), sl = pin(st[k]), sh = pin(st[4 + k]);
-    if (q == k) { r_lo = rl; r_hi = rh; a = ak; s_lo = sl; s_hi = sh; }
-  }
-  gmem(rec)[q] = r_lo;
-  gmem(rec)[4 + q] = r_hi;
-  gmem(rec)[8 + q] = a;
-  st_out[q] = s_lo;
-  st_out[4 + q] = s_hi;
-  if (q == 0) st_out[8] = st[8];
-  if constexpr (!std::is_same_v<AlphaPtr, std::nullptr_t>) alpha_out[q] = a;
+  gmem(rec)[8 + q] = alpha;
+  return alpha;
 }
 
 }  // namespace
@@ -219,9 +224,12 @@ __global__ void __launch_bounds__(256) fri_layer_kernel(FriLayerDesc d, uint32_t
                                                         uint32_t* __restrict__ ticket) {
   __shared__ __align__(16) uint32_t bufA[8 << 10];
   __shared__ __align__(16) uint32_t bufB[8 << 9];
+  __shared__ QuadBufs quads;
+  __shared__ uint32_t ch[16];
   __shared__ uint32_t last;
   const uint32_t t = threadIdx.x, w = blockIdx.x;
   const uint32_t l = d.log, C = 1u << c;
+  const QuadSchedule sched = quad_schedule(t >> 2, t & 3);
   qm31 alpha = qm_zero();
   if (d.mode != FRI_LEAVES) alpha = {gmem(d.alpha)[0], gmem(d.alpha)[1], gmem(d.alpha)[2], gmem(d.alpha)[3]};
   for (uint32_t r = t; r < C; r += FL_THREADS) {
@@ -229,13 +237,11 @@ __global__ void __launch_bounds__(256) fri_layer_kernel(FriLayerDesc d, uint32_t
     const qm31 v = fri_value_global(d, i, alpha);
     uint32_t h[8];
     leaf_hash(v, h);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) bufA[k * C + r] = h[k];
+    fl_put(bufA, quads, C, r, h);
     store8(d.nodes + 8 * (((size_t)1 << l) - 1 + i), h);
   }
   __syncthreads();
-  const uint32_t* top = fl_levels(bufA, bufB, C, l, w * C, d.nodes);
-  uint32_t root[8];
+  const uint32_t* top = fl_levels(bufA, bufB, quads, sched, C, l, w * C, d.nodes);
   if (gridDim.x > 1) {
     // The chunk root is published with device-scope atomic exchanges, which are performed where
     // every XCD reads them; wave 0 waits for their results before it takes the ticket. This orders
@@ -261,20 +267,19 @@ __global__ void __launch_bounds__(256) fri_layer_kernel(FriLayerDesc d, uint32_t
       uint32_t r[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) r[k] = __hip_atomic_fetch_or(g + 8 * i + k, zero, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) bufA[k * R + i] = r[k];
+      fl_put(bufA, quads, R, i, r);
     }
     __syncthreads();
-    top = fl_levels(bufA, bufB, R, lev, 0, d.nodes);
+    top = fl_levels(bufA, bufB, quads, sched, R, lev, 0, d.nodes);
   }
   if (t < 4) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) root[k] = top[k];
-    uint32_t st[9], a[4];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) st[k] = d.init ? d.st0[k] : state[k];
-    fl_channel(st, root, t, a);
-    fl_publish(t, st, root, a, d.rec, state, nullptr);
+    ch[t] = d.init ? d.st0[t] : state[t];
+    ch[4 + t] = d.init ? d.st0[4 + t] : state[4 + t];
+    fl_channel(ch, top, sched, t, d.rec);
+    quad_sync();
+    state[t] = ch[t];
+    state[4 + t] = ch[4 + t];
+    if (t == 0) state[8] = ch[8];
     if (d.init && t < 2) state[14 + t] = ~0u;
   }
 }
@@ -287,10 +292,11 @@ __global__ void __launch_bounds__(256) fri_small_kernel(const FriLayerDesc* __re
                                                         uint32_t* __restrict__ state) {
   __shared__ uint32_t V[4][256];
   __shared__ __align__(16) uint32_t bufA[8 << 8];
-  __shared__ __align__(16) uint32_t bufB[8 << 7];
-  __shared__ uint32_t st_s[9], alpha_s[4];
+  __shared__ QuadBufs quads;
+  __shared__ uint32_t ch[16], alpha_s[4];
   const uint32_t t = threadIdx.x;
-  if (t < 9) st_s[t] = state[t];
+  const QuadSchedule sched = quad_schedule(t >> 2, t & 3);
+  if (t < 9) ch[t] = state[t];
   __syncthreads();
   for (uint32_t e = 0; e < n; ++e) {
     const FriLayerDesc d = descs[e];
@@ -319,8 +325,7 @@ __global__ void __launch_bounds__(256) fri_small_kernel(const FriLayerDesc* __re
       if (t < N) {
         uint32_t h[8];
         leaf_hash(v, h);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) bufA[k * N + t] = h[k];
+        fl_put(bufA, quads, N, t, h);
         store8(d.nodes + 8 * ((size_t)N - 1 + t), h);
       }
     } else {
@@ -330,26 +335,19 @@ __global__ void __launch_bounds__(256) fri_small_kernel(const FriLayerDesc* __re
         uint32_t hA, hB;
         blake2s_init_quad(q, hA, hB);
         blake2s_compress_quad(hA, hB, msg, 16, true, q);
-        bufA[q * N + p] = hA;
-        bufA[(4 + q) * N + p] = hB;
+        const uint32_t o = quad_node(p);
+        quads.a[o + q] = hA;
+        quads.a[o + 4 + q] = hB;
         gmem(d.nodes)[8 * (N - 1 + p) + q] = hA;
         gmem(d.nodes)[8 * (N - 1 + p) + 4 + q] = hB;
       }
     }
     __syncthreads();
-    const uint32_t* top = fl_levels(bufA, bufB, N, d.log, 0, d.nodes);
-    if (t < 4) {
-      uint32_t root[8], st[9], a[4];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) root[k] = top[k];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) st[k] = st_s[k];
-      fl_channel(st, root, t, a);
-      fl_publish(t, st, root, a, d.rec, st_s, alpha_s);
-    }
+    const uint32_t* top = fl_levels(bufA, nullptr, quads, sched, N, d.log, 0, d.nodes);
+    if (t < 4) alpha_s[t] = fl_channel(ch, top, sched, t, d.rec);
     __syncthreads();
   }
-  if (t < 9) state[t] = st_s[t];
+  if (t < 9) state[t] = ch[t];
 }
 
 // The last layer's interpolation, the channel mix of the last polynomial and the proof-of-work

@@ -160,43 +160,41 @@ void launch_merkle_layer_small(uint32_t log_size, const uint32_t* prev, const ui
 // Up to 9 levels of a Merkle tree with no injected columns in one launch. Workgroup w reads the
 // 2^L children [w 2^L, (w+1) 2^L) of level log_child and writes its 2^(L-j) nodes of level
 // log_child - j (j = 1..L); the levels in between stay in LDS. The levels are latency-bound (each
-// waits for the one below), so every node is hashed by a quad of lanes (blake2s_compress_quad):
+// waits for the one below), so every node is hashed by a quad of lanes (blake2s_compress_quad_lds):
 // 4 * 2^(L-1) threads, lane q of a quad holding chaining words q and 4 + q.
-constexpr uint32_t SUBTREE_MAX_LEVELS = 9;
+constexpr uint32_t SUBTREE_MAX_LEVELS = 9, SUBTREE_QUADS = 1u << (SUBTREE_MAX_LEVELS - 1);
 struct LayerPtrs { uint32_t* p[SUBTREE_MAX_LEVELS]; };
 __global__ void __launch_bounds__(1024) merkle_subtree_kernel(const uint32_t* __restrict__ child, uint32_t L,
                                                               LayerPtrs outs) {
   CRITICAL_PATH_WAVE();
-  __shared__ uint32_t lds[(1u << (SUBTREE_MAX_LEVELS - 1)) * 8];
+  __shared__ uint32_t even[SUBTREE_QUADS * QUAD_MSG], odd[SUBTREE_QUADS / 2 * QUAD_MSG];
   const uint32_t w = blockIdx.x, nd = threadIdx.x >> 2, q = threadIdx.x & 3;
-  uint32_t n = 1u << (L - 1);  // nodes of the first level computed by this workgroup
-  for (uint32_t j = 0; j < L; ++j, n >>= 1) {
-    uint32_t hA = 0, hB = 0;
+  const QuadSchedule sched = quad_schedule(nd, q);
+  uint32_t n = 1u << (L - 1);  // nodes of the level to compute
+  if (nd < n) {  // a quad reads its own message
+    const uint4 v = reinterpret_cast<const uint4*>(child + ((size_t)w * n + nd) * 16)[q];
+    uint32_t* m = even + nd * QUAD_MSG + 4 * q;
+    m[0] = v.x; m[1] = v.y; m[2] = v.z; m[3] = v.w;
+    quad_sync();
+  }
+  const auto level = [&](const uint32_t* in, uint32_t* out, uint32_t* o) {
     if (nd < n) {
-      uint32_t m[16];
-      if (j == 0) {
-        const uint4* p4 = reinterpret_cast<const uint4*>(child + ((size_t)w * 2 * n + 2 * nd) * 8);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint4 v = p4[k];
-          m[4 * k] = v.x; m[4 * k + 1] = v.y; m[4 * k + 2] = v.z; m[4 * k + 3] = v.w;
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < 16; ++k) m[k] = lds[2 * nd * 8 + k];
-      }
+      uint32_t hA, hB;
       blake2s_init_quad(q, hA, hB);
-      blake2s_compress_quad(hA, hB, m, 64, true, q);
-    }
-    __syncthreads();
-    if (nd < n) {
-      lds[nd * 8 + q] = hA;
-      lds[nd * 8 + 4 + q] = hB;
-      uint32_t* o = outs.p[j] + ((size_t)w * n + nd) * 8;
+      blake2s_compress_quad_lds(hA, hB, in, sched, 64, true, q);
+      const uint32_t at = quad_node(nd);
+      out[at + q] = hA;
+      out[at + 4 + q] = hB;
+      o += ((size_t)w * n + nd) * 8;
       o[q] = hA;
       o[4 + q] = hB;
     }
+    n >>= 1;
     __syncthreads();
+  };
+  for (uint32_t j = 0; j < L; j += 2) {  // the two buffers are named, so that their addresses are constants
+    level(even, odd, outs.p[j]);
+    if (j + 1 < L) level(odd, even, outs.p[j + 1]);
   }
 }
 
