@@ -216,7 +216,8 @@ int stwo_hip_copy_h2d(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_
 }
 int stwo_hip_copy_d2h(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_t n) {
   return guarded(h, [&](Ctx& c) {
-    // memory that is not a whole column of this context (any other is the copy engine's to judge)
+    // the start of a column of this context may be read by a kernel; any other address goes to the copy
+    // engine, which checks it
     const auto it = c.col_live.find(const_cast<uint32_t*>(src));
     c.d2h(dst, src, n * 4, it != c.col_live.end() && it->second >= n * 4);
   });
