@@ -478,11 +478,14 @@ __global__ void __launch_bounds__(256) accumulate_lifts_kernel(uint32_t n_quads,
                                                                uint32_t n_src) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_quads) return;
+  // every load is ahead of the first store: a source may hold the destination's columns in another order
+  u32x4 v[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    u32x4 v = ld4(base.c[k], 4 * i);
-    for (uint32_t s = 0; s < n_src; ++s) {
-      const uint32_t r = a.s[s].r;
+  for (int k = 0; k < 4; ++k) v[k] = ld4(base.c[k], 4 * i);
+  for (uint32_t s = 0; s < n_src; ++s) {
+    const uint32_t r = a.s[s].r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
       u32x4 x;
       if (r == 0) {
         x = ld4(a.s[s].c[k], 4 * i);
@@ -491,10 +494,11 @@ __global__ void __launch_bounds__(256) accumulate_lifts_kernel(uint32_t n_quads,
         x = u32x4{p.x, p.y, p.x, p.y};
       }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = m31_add(v[q], x[q]);
+      for (int q = 0; q < 4; ++q) v[k][q] = m31_add(v[k][q], x[q]);
     }
-    st4(dst.c[k], 4 * i, v);
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) st4(dst.c[k], 4 * i, v[k]);
 }
 // One source, any alignment and size, added in place.
 __global__ void __launch_bounds__(256) accumulate_lifted_kernel(uint32_t log_dst, Cols4 dst, uint32_t log_src,

@@ -1,5 +1,6 @@
 """AccumulationOps in one pass: sums of lifted secure columns of many sizes (more than one launch's
-sources among them), equal sizes, the smallest ones, and columns off the vector form's alignment, against the
+sources among them), equal sizes, the smallest ones, columns off the vector form's alignment, and a source that
+holds the destination's own columns, against the
 definition out[i] = sum over the columns of col[(i >> (r + 1) << 1) + (i & 1)], r the difference of the log
 sizes; and the sums of block results in out-of-domain evaluation, from one block to several waves' worth."""
 import numpy as np
@@ -42,6 +43,20 @@ def test_lift_and_accumulate(hb, logs, off):
                                                   SH._ptrs([c.ptr + 4 * off for c in out])))
     for k in range(4):
         assert np.array_equal(out[k].to_cpu()[off:], (exp[k] % P).astype(np.uint32))
+
+
+@pytest.mark.parametrize("log_size", [0, 1, 2, 7, 10])
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("order", [(0, 1, 2, 3), (1, 2, 3, 0), (0, 0, 0, 0)])
+def test_accumulate_of_its_own_coordinates(hb, log_size, off, order):
+    """The source holds the destination's columns, in any order: every sum is of the old values."""
+    print("accumulate own", log_size, off, order, flush=True)
+    data = np.random.default_rng(log_size).integers(0, P, (4, 1 << log_size), dtype=np.uint64)
+    cols = [hb.from_cpu(np.concatenate([np.zeros(off, np.uint32), c.astype(np.uint32)])) for c in data]
+    dst = SH._ptrs([c.ptr + 4 * off for c in cols])
+    hb._check(hb.lib.stwo_hip_accumulate(hb.ctx, log_size, dst, SH._ptrs([cols[k].ptr + 4 * off for k in order])))
+    for k in range(4):
+        assert np.array_equal(cols[k].to_cpu()[off:], ((data[k] + data[order[k]]) % P).astype(np.uint32)), k
 
 
 @pytest.mark.parametrize("log_size", [3, 11, 12, 17, 19])
