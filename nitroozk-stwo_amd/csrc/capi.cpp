@@ -215,12 +215,7 @@ int stwo_hip_copy_h2d(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_
   });
 }
 int stwo_hip_copy_d2h(stwo_hip_ctx* h, uint32_t* dst, const uint32_t* src, size_t n) {
-  return guarded(h, [&](Ctx& c) {
-    // the start of a column of this context may be read by a kernel; any other address goes to the copy
-    // engine, which checks it
-    const auto it = c.col_live.find(const_cast<uint32_t*>(src));
-    c.d2h(dst, src, n * 4, it != c.col_live.end() && it->second >= n * 4);
-  });
+  return guarded(h, [&](Ctx& c) { c.read_column(dst, src, 0, n); });
 }
 static_assert(GATHER_ARG_COLS * GATHER_ARG_ROWS <= Ctx::gather_host_words,
               "an argument-block gather must fit the coherent host buffer");
@@ -252,7 +247,7 @@ int stwo_hip_batch_at_multi(stwo_hip_ctx* h, const uint32_t* const* cols, uint32
       const std::vector<uint32_t> rv(rows, rows + n_rows);
       launch_gather_rows(c.table_vec(bases), n_cols, c.upload_vec(rv), n_rows, o, c.stream);
     }
-    c.d2h(out_host, o, n * 4);
+    c.read_own(out_host, o, n * 4);
     c.reset_arena();
   });
 }
@@ -266,11 +261,11 @@ int stwo_hip_precompute_twiddles(stwo_hip_ctx* h, uint32_t log_domain, uint32_t*
     size_t off = c.tree_len() - n;
     if (tw) {
       std::vector<uint32_t> t(n);
-      c.d2h(t.data(), c.tw.p + off, n * 4);
+      c.read_own(t.data(), c.tw.p + off, n * 4);
       // layers of the smaller tree are the last layers of the larger tree, followed by the pad
       memcpy(tw, t.data(), n * 4);
     }
-    if (itw) c.d2h(itw, c.itw.p + off, n * 4);
+    if (itw) c.read_own(itw, c.itw.p + off, n * 4);
   });
 }
 
@@ -328,7 +323,7 @@ int stwo_hip_batch_eval_at_point(stwo_hip_ctx* h, const uint32_t* const* coeffs,
     c.commit_staged();
     launch_oods(d_tasks, d_tg, n_cols, d_bs, (uint32_t)bs.size() - 1, log_size, d_f, d_gl, 1, (qm31*)w.p,
                 (qm31*)partials.p, (qm31*)vals.p, c.stream);
-    c.d2h(out_host, vals.p, (size_t)n_cols * 16);
+    c.read_own(out_host, vals.p, (size_t)n_cols * 16);
     c.reset_arena();
   });
 }
@@ -379,7 +374,7 @@ int stwo_hip_batch_eval_at_point_noalloc(stwo_hip_ctx* h, const uint32_t* const*
     c.commit_staged();
     launch_oods(d_tasks, d_tg, n_cols, d_bs, (uint32_t)bs.size() - 1, log_size, d_f, d_gl, 1, w, partials, vals,
                 c.stream);
-    c.d2h(out_host, vals, (size_t)n_cols * 16);
+    c.read_own(out_host, vals, (size_t)n_cols * 16);
     c.reset_arena();
   }, /*may_recycle=*/false);
 }
@@ -417,7 +412,7 @@ int stwo_hip_batch_barycentric_eval(stwo_hip_ctx* h, const uint32_t* const* eval
     launch_barycentric_eval(log_size, (const uint32_t* const*)c.upload_vec(ev), n_cols,
                             {{weights[0], weights[1], weights[2], weights[3]}}, (qm31*)partial.p, (qm31*)vals.p,
                             c.stream);
-    c.d2h(out_host, vals.p, (size_t)n_cols * 16);
+    c.read_own(out_host, vals.p, (size_t)n_cols * 16);
     c.reset_arena();
   });
 }
@@ -1003,7 +998,7 @@ int stwo_hip_gen_interaction_trace_poseidon(stwo_hip_ctx* h, const uint32_t* con
                               (const unsigned long long*)sums.p, scratch.p, c.stream);
     }
     unsigned long long sv[4];
-    c.d2h(sv, sums.p, sizeof(sv));
+    c.read_own(sv, sums.p, sizeof(sv));
     *claimed_sum = {m31_reduce64(sv[0] % P), m31_reduce64(sv[1] % P), m31_reduce64(sv[2] % P), m31_reduce64(sv[3] % P)};
     c.reset_arena();
   });
@@ -1122,7 +1117,7 @@ int stwo_hip_bit_reverse_column(stwo_hip_ctx* h, uint32_t* col, uint32_t log_siz
 int stwo_hip_column_at(stwo_hip_ctx* h, const uint32_t* col, size_t index, uint32_t* out) {
   return guarded(h, [&](Ctx& c) {
     if (!col || !out) throw HipError(1, "null argument");
-    c.d2h(out, col + index, 4);
+    c.read_column(out, col, index, 1);
   });
 }
 int stwo_hip_column_set(stwo_hip_ctx* h, uint32_t* col, size_t index, uint32_t value) {
@@ -1171,8 +1166,8 @@ int stwo_hip_twiddles_read(stwo_hip_ctx* h, const stwo_hip_twiddles* t, uint32_t
   return guarded(h, [&](Ctx& c) {
     if (!t || !h->trees.count(const_cast<stwo_hip_twiddles*>(t))) throw HipError(1, "unknown twiddle tree");
     const size_t n = (size_t)1 << t->log_size;
-    if (tw_host) c.d2h(tw_host, t->tw.p, n * 4);
-    if (itw_host) c.d2h(itw_host, t->itw.p, n * 4);
+    if (tw_host) c.read_own(tw_host, t->tw.p, n * 4);
+    if (itw_host) c.read_own(itw_host, t->itw.p, n * 4);
   });
 }
 int stwo_hip_twiddles_free(stwo_hip_ctx* h, stwo_hip_twiddles* t) {
@@ -1246,7 +1241,7 @@ int stwo_hip_eval_at_point_by_folding(stwo_hip_ctx* h, const uint32_t* evals, ui
       alpha = qm_double_x(alpha);
     }
     uint32_t v[4];
-    for (int k = 0; k < 4; ++k) c.d2h(&v[k], cur.c[k], 4);
+    for (int k = 0; k < 4; ++k) c.read_own(&v[k], cur.c[k], 4);
     const qm31 r = qm_mul_m31({v[0], v[1], v[2], v[3]}, m31_inv(1u << log_size));
     *out = q(r);
   });
@@ -1307,7 +1302,7 @@ int stwo_hip_channel_grind(stwo_hip_ctx* h, uint32_t* state, uint32_t pow_bits, 
     }
     if (c.capturing) return;
     unsigned long long found = ~0ull;
-    c.d2h(&found, st + 10, 8);
+    c.read_own(&found, st + 10, 8);
     // beyond the first range: further launches on the device prefix, doubling, as device_grind
     const uint64_t limit = (uint64_t)0x7fffffff << 20;
     for (uint64_t start = count; found == ~0ull; start += count) {
@@ -1315,7 +1310,7 @@ int stwo_hip_channel_grind(stwo_hip_ctx* h, uint32_t* state, uint32_t pow_bits, 
       count = count < (1u << 24) ? count * 2 : count;
       launch_grind_dev(st + 12, pow_bits, start, (uint32_t)count, reinterpret_cast<unsigned long long*>(st + 10),
                        c.stream);
-      c.d2h(&found, st + 10, 8);
+      c.read_own(&found, st + 10, 8);
     }
     const uint32_t w[2] = {(uint32_t)found, (uint32_t)(found >> 32)};
     HIP_CHECK(hipMemcpyAsync(nonce, w, 8, hipMemcpyHostToDevice, c.stream));
@@ -1326,7 +1321,7 @@ int stwo_hip_channel_read(stwo_hip_ctx* h, const uint32_t* state, uint8_t digest
   return guarded(h, [&](Ctx& c) {
     if (!state || !digest || !n_draws) throw HipError(1, "null argument");
     uint32_t w[9];
-    c.d2h(w, state, sizeof(w));
+    c.read_column(w, state, 0, 9);
     for (int i = 0; i < 8; ++i)
       for (int j = 0; j < 4; ++j) digest[4 * i + j] = (uint8_t)(w[i] >> (8 * j));
     *n_draws = w[8];

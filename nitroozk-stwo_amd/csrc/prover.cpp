@@ -60,7 +60,7 @@ thread_local HostMarks g_marks;
 
 Hash read_hash(Ctx& ctx, const uint32_t* dev) {
   uint32_t w[8];
-  ctx.d2h(w, dev, 32);
+  ctx.read_own(w, dev, 32);
   Hash h;
   for (int i = 0; i < 8; ++i)
     for (int j = 0; j < 4; ++j) h[4 * i + j] = (uint8_t)(w[i] >> (8 * j));
@@ -286,7 +286,7 @@ uint64_t device_grind(Ctx& ctx, const Hash& prefix, uint32_t pow_bits, unsigned 
       KScope ks(ctx, K_GRIND, 0.0);
       launch_grind(pre, pow_bits, start, (uint32_t)count, slot, ctx.stream);
     }
-    ctx.d2h(&found, slot, 8);
+    ctx.read_own(&found, slot, 8);
   }
   return found;
 }
@@ -1192,7 +1192,7 @@ int prove_ex(Ctx& ctx, Channel& ch, std::vector<DevTree>& trees, const std::vect
   HMARK("x_friprep");
 
   // the uploads above stay in the staging arena until the quotient kernels have run
-  if (n_vals) ctx.d2h(S.val.data(), dvals_p, n_vals * 16);
+  if (n_vals) ctx.read_own(S.val.data(), dvals_p, n_vals * 16);
   HMARK("oods_gpu");
   ch.mix_felts(S.val);
   HMARK("oods_post");
@@ -1328,7 +1328,7 @@ int prove_ex(Ctx& ctx, Channel& ch, std::vector<DevTree>& trees, const std::vect
       if (cur.c[k].p != dlast + k * last_n) launch_copy_words(dlast + k * last_n, cur.c[k].p, last_n, ctx.stream);
     // the whole block: channel state and proof-of-work slot, records, last layer, prefix
     fri_hb.assign(16 + 12 * (size_t)n_layers + 4 * last_n + 8, 0);
-    ctx.d2h(fri_hb.data(), dstate, fri_hb.size() * 4);
+    ctx.read_own(fri_hb.data(), dstate, fri_hb.size() * 4);
     const uint32_t* hb = fri_hb.data() + 16;
     ctx.reset_arena();
     HMARK("fri_wait");
@@ -1596,7 +1596,7 @@ ProveResult prove_poseidon(Ctx& ctx, const std::vector<const uint32_t*>& trace, 
     comps.assign(1, c);
     prepare_composition(ctx, trees, comps, prep);
     uint32_t w[16];
-    ctx.d2h(w, sums.p, sizeof(w));
+    ctx.read_own(w, sums.p, sizeof(w));
     unsigned long long s[4];
     std::memcpy(s, w, sizeof(s));
     c.claimed_sum = {m31_reduce64(s[0] % P), m31_reduce64(s[1] % P), m31_reduce64(s[2] % P), m31_reduce64(s[3] % P)};

@@ -356,15 +356,18 @@ void* Ctx::readback_buf(size_t bytes) {
   }
   return rb_pinned;
 }
-void Ctx::d2h(void* dst, const void* src, size_t bytes, bool by_kernel) {
-  if (by_kernel && bytes && bytes <= READ_WORDS * 4 && (bytes | (uintptr_t)src) % 4 == 0) {
-    commit_staged();
-    launch_read_words((const uint32_t*)src, (uint32_t)(bytes / 4), gather_host_dev, gather_flag(), ++gather_call,
-                      stream);
-    wait_gather();
-    std::memcpy(dst, gather_host, bytes);
-    return;
-  }
+void Ctx::read_column(void* dst, const uint32_t* col, size_t first, size_t words) {
+  if (kernel_may_read(col_live, col, first, words)) read_own(dst, col + first, words * 4);
+  else d2h(dst, col + first, words * 4);
+}
+void Ctx::read_own(void* dst, const void* src, size_t bytes) {
+  if (!bytes || bytes > READ_WORDS * 4 || (bytes | (uintptr_t)src) % 4) return d2h(dst, src, bytes);
+  commit_staged();
+  launch_read_words((const uint32_t*)src, (uint32_t)(bytes / 4), gather_host_dev, gather_flag(), ++gather_call, stream);
+  wait_gather();
+  std::memcpy(dst, gather_host, bytes);
+}
+void Ctx::d2h(void* dst, const void* src, size_t bytes) {
   // through pinned memory: a read-back into pageable memory goes through the runtime's own
   // staging, which costs tens of microseconds more per call
   if (bytes <= d2h_cap) {
@@ -396,7 +399,7 @@ void build_twiddle_tree(Ctx& c, uint32_t init_index, uint32_t log_size, DevBuf& 
   launch_twiddle_tree(init_index, log_size, tw.p, itw.p, tw2.p, itw2.p, (double*)twd.p, (double*)itwd.p,
                       flag.p, c.stream);
   uint32_t zero = 0;
-  c.d2h(&zero, flag.p, 4);
+  c.read_own(&zero, flag.p, 4);
   if (zero) throw HipError(1, "the coset has a point with x = 0, whose twiddle has no inverse");
 }
 

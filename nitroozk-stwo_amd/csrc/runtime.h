@@ -13,6 +13,7 @@
 #include "blake2s.h"
 #include "field.h"
 #include "kernels.h"
+#include "read_route.h"
 
 namespace sh {
 
@@ -103,7 +104,7 @@ struct Ctx {
   // shapes makes no allocator calls after its first request. Cached bytes are capped.
   void* col_alloc(size_t bytes);
   void col_free(void* p);
-  std::unordered_map<void*, size_t> col_live;
+  LiveColumns col_live;
   std::unordered_map<size_t, std::vector<void*>> col_cache;
   size_t col_cached_bytes = 0;
   static constexpr size_t COL_CACHE_CAP = (size_t)32 << 30;
@@ -189,9 +190,13 @@ struct Ctx {
   int cu_count = 0;
   const uint32_t* domain_xy(uint32_t log);
   uint32_t tree_len() const { return 1u << (tw_log - 1); }
-  // Synchronous. by_kernel: src is known to be device memory that a kernel may read, so a short read
-  // may take launch_read_words.
-  void d2h(void* dst, const void* src, size_t bytes, bool by_kernel = true);
+  // Synchronous copies to the host. d2h goes through the copy engine, which refuses an address that is not
+  // memory it knows: the one for addresses that a caller gave. read_own is for buffers of this context,
+  // whose short reads a kernel may do; read_column for `words` words from word `first` of what a caller
+  // says is a column: by a kernel only where kernel_may_read finds them in one.
+  void d2h(void* dst, const void* src, size_t bytes);
+  void read_own(void* dst, const void* src, size_t bytes);
+  void read_column(void* dst, const uint32_t* col, size_t first, size_t words);
   // Coherent pinned host memory that small gathers write directly from the device (zero copy),
   // and behind it the flag that takes a gather's call number when its words are there.
   uint32_t* gather_host = nullptr;

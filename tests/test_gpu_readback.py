@@ -1,7 +1,9 @@
 """Small reads of device memory (batch_at_multi within the argument block, copy_d2h of a column's first
 words), which the host awaits by a flag: every size where the route changes, addresses inside a column
-and alignment, many reads in a row with work between them that outlasts the polling, and reads
-interleaved over two contexts on two threads, each against the same words kept on the host."""
+and alignment, single words by every route, many reads in a row with work between them that outlasts the
+polling, and reads interleaved over two contexts on two threads, each against the same words kept on the
+host."""
+import ctypes
 import threading
 
 import numpy as np
@@ -40,6 +42,30 @@ def test_reads(hb, n):
         out = np.full(n, 7, np.uint32)
         hb._check(hb.lib.stwo_hip_copy_d2h(hb.ctx, out.ctypes.data, col.ptr + 4 * off, n))
         assert (out == data[off:off + n]).all()
+
+
+@pytest.mark.parametrize("n", [1, 9, 64, 5000])
+def test_single_words_by_every_route(hb, n):
+    """column_at and channel_read of a column's own address (a kernel reads it) and of addresses that are
+    not one of the context's columns: inside a column, and another context's."""
+    print("column_at", n, flush=True)
+    data = np.random.default_rng(n).integers(0, 1 << 32, n + 1, dtype=np.uint64).astype(np.uint32)
+    other = SH.HipBackend(0)
+    try:
+        mine, theirs = hb.from_cpu(data), other.from_cpu(data)
+        other.synchronize()
+        word = np.zeros(1, np.uint32)
+        digest, draws = ctypes.create_string_buffer(32), ctypes.c_uint32()
+        for base in (mine.ptr, theirs.ptr):
+            for off in (0, 1):
+                for i in sorted({0, n // 2, n - off}):
+                    hb._check(hb.lib.stwo_hip_column_at(hb.ctx, base + 4 * off, i, word.ctypes.data_as(SH._U32P)))
+                    assert word[0] == data[off + i]
+                if n >= 9:
+                    hb._check(hb.lib.stwo_hip_channel_read(hb.ctx, base + 4 * off, digest, ctypes.byref(draws)))
+                    assert digest.raw == data[off:off + 8].tobytes() and draws.value == data[off + 8]
+    finally:
+        other.close()
 
 
 def test_reads_behind_long_work(hb):
