@@ -425,10 +425,14 @@ int stwo_hip_commit_on_layer(stwo_hip_ctx* h, uint32_t log_size, const uint32_t*
     // columns laid out at a fixed stride of one column need no address table
     bool strided = n_cols > 1;
     for (uint32_t k = 1; strided && k < n_cols; ++k) strided = v[k] == v[0] + ((size_t)k << log_size);
-    // at most 16 columns travel as kernel arguments (no staged table; under graph capture the only way)
-    const bool small = n_cols <= 16;
-    if (c.capturing && !strided && !small) throw HipError(3, "not capturable: more than 16 columns not at one stride");
-    const uint32_t* const* d = !strided && !small ? (const uint32_t* const*)c.upload_vec(v) : nullptr;
+    // 1 to 16 columns travel as kernel arguments. Columns at one stride could take the pipelined leaf kernel
+    // instead: it gains from 9 columns of 2^20 rows (16 of them 33.8 us against 36.7), and loses on 4 to 8 at
+    // any size (4 of 2^20 33.9 against 31.4, of 2^22 122 against 111), on 9 to 12 of 2^22 (126 against 119 to
+    // 124), and up to 2^14 rows both are the launch. Children alone need no columns: 170 such layers of an
+    // FRI commitment 4.7 us a call, 5.1 with an empty argument block (2^21: 61.3 and 62.1).
+    const bool small = n_cols != 0 && n_cols <= 16;
+    if (c.capturing && n_cols > 16 && !strided) throw HipError(3, "not capturable: more than 16 columns not at one stride");
+    const uint32_t* const* d = n_cols > 16 && !strided ? (const uint32_t* const*)c.upload_vec(v) : nullptr;
     {
       KScope ks(c, K_MERKLE, ((prev ? 64.0 : 0.0) + 4.0 * n_cols + 32.0) * (double)(1u << log_size));
       ks.units(blake2s_node_compressions(prev != nullptr, n_cols) * (double)(1u << log_size));

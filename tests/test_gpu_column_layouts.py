@@ -1,7 +1,7 @@
 """How a call's columns lie in memory never changes its results: rows of one allocation (no address
 table), the same rows backwards, one source column given several times, scattered columns, columns at an
 odd distance, and more columns than a launch's arguments hold, against the oracle. Transforms in one
-kernel, in several passes and below the LDS kernels' sizes; Merkle layers of 1..17 and 40 columns on both
+kernel, in several passes and below the LDS kernels' sizes; Merkle layers of 0..17 and 40 columns on both
 sides of the 16 that travel as arguments."""
 import numpy as np
 import pytest
@@ -67,7 +67,7 @@ def test_one_source_for_every_column(hb):
     assert np.array_equal(out.to_cpu(), np.tile(exp, n))
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 40])
+@pytest.mark.parametrize("n", [0, 1, 2, 15, 16, 17, 40])
 @pytest.mark.parametrize("with_prev", [False, True])
 def test_merkle_layers(hb, n, with_prev):
     log_n = 5
