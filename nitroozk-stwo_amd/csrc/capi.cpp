@@ -100,7 +100,7 @@ void run_fft(Ctx& c, bool inverse, const uint32_t* const* src, uint32_t* const* 
   }
   const ColSet ds = c.col_set(src, n_cols, false), dd = c.col_set((const uint32_t* const*)dst, n_cols, false);
   c.commit_staged();
-  launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, c.stream, false, low);
+  launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, c.cu_count, c.stream, false, low);
 }
 uint32_t plan_fft(Ctx& c, bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree) {
   return log_n <= 2 ? 0u : c.fft_low_log(inverse, n_cols, log_in, log_n, tree);

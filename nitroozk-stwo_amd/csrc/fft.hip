@@ -526,10 +526,8 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(ColSet src, ColSet
 // grid that holds every CU until the transform is done doubled the time of the trace's Merkle tree).
 template <bool INV, int S>
 static void launch_low_tile(uint32_t n_cols, ColSet src, ColSet dst, uint32_t log_n,
-                            uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
-  int dev = 0, cus = 0;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+                            uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, int cus,
+                            hipStream_t stream) {
   const uint32_t n_tiles = n_cols << (log_n - S), resident = (uint32_t)(cus > 8 ? cus / 8 * 8 : 8) << (15 - S);
   const uint32_t grid = prio && n_tiles > resident ? resident : n_tiles;
   hipLaunchKernelGGL((fft_low_kernel<INV, S>), dim3(grid), dim3(LOW_T<S>), 0, stream, src, dst, log_n, in_mask,
@@ -537,13 +535,13 @@ static void launch_low_tile(uint32_t n_cols, ColSet src, ColSet dst, uint32_t lo
 }
 template <bool INV>
 static void launch_low(uint32_t S, uint32_t n_cols, ColSet src, ColSet dst, uint32_t log_n,
-                       uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, hipStream_t stream) {
+                       uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, int cus, hipStream_t stream) {
   switch (S) {
-    case 11: return launch_low_tile<INV, 11>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
-    case 12: return launch_low_tile<INV, 12>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
-    case 13: return launch_low_tile<INV, 13>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
-    case 14: return launch_low_tile<INV, 14>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
-    default: return launch_low_tile<INV, 15>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, stream);
+    case 11: return launch_low_tile<INV, 11>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, cus, stream);
+    case 12: return launch_low_tile<INV, 12>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, cus, stream);
+    case 13: return launch_low_tile<INV, 13>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, cus, stream);
+    case 14: return launch_low_tile<INV, 14>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, cus, stream);
+    default: return launch_low_tile<INV, 15>(n_cols, src, dst, log_n, in_mask, tree, rot, prio, cus, stream);
   }
 }
 
@@ -570,7 +568,7 @@ static std::vector<FftPass> plan_passes(uint32_t k, uint32_t K) {
 }
 
 void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t log_in,
-                uint32_t log_n, const FftTree& ft, hipStream_t stream, bool background, uint32_t low_log) {
+                uint32_t log_n, const FftTree& ft, int cus, hipStream_t stream, bool background, uint32_t low_log) {
   if (n_cols == 0) return;
   const uint32_t prio = background ? 0u : 1u;
   const uint32_t* const tree = ft.t2;
@@ -627,7 +625,7 @@ void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t 
     }
     if (inverse) {
       // 2^-log_n is 2^(31 - log_n): the low stages' own scaling is a rotation
-      launch_low<true>(S, n_cols, src, dst, log_n, full, ft, high.empty() ? 31 - log_n : 0u, prio, stream);
+      launch_low<true>(S, n_cols, src, dst, log_n, full, ft, high.empty() ? 31 - log_n : 0u, prio, cus, stream);
       for (size_t i = 0; i < high.size(); ++i)
         run_pass(high[i], dst, full, i + 1 == high.size() ? inv_n : 0u);
     } else {
@@ -635,7 +633,7 @@ void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t 
         run_pass(high[ii], ii + 1 == high.size() ? src : dst,
                  ii + 1 == high.size() ? in_mask : full, 0u);
       launch_low<false>(S, n_cols, high.empty() ? src : dst, dst, log_n,
-                        high.empty() ? in_mask : full, ft, 0u, prio, stream);
+                        high.empty() ? in_mask : full, ft, 0u, prio, cus, stream);
     }
     return;
   }

@@ -143,11 +143,11 @@ uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32
   for (uint32_t s = 11; s <= smax; ++s) cand.push_back(s);
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
   for (uint32_t c : cand) {
-    launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, stream, background, c);  // warm-up
+    launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, cu_count, stream, background, c);  // warm-up
     for (int rep = 0; rep < 2; ++rep) {
       hipEvent_t a = get_event(), b = get_event();
       HIP_CHECK(hipEventRecord(a, stream));
-      launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, stream, background, c);
+      launch_fft(inverse, ds, dd, n_cols, log_in, log_n, tree, cu_count, stream, background, c);
       HIP_CHECK(hipEventRecord(b, stream));
       ev.push_back({a, b});
     }

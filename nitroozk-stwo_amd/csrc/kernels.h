@@ -22,7 +22,7 @@ struct FftTree {
   uint32_t len;
 };
 inline size_t fft_tree_doubles(size_t len) { return len < 16 ? 1 : len / 16; }
-// background: the transform runs beside critical-path kernels on another stream and leaves them the
+// cus: the device's compute units. background: the transform runs beside critical-path kernels on another stream and leaves them the
 // issue priority, and CUs as its tiles end. low_log: the tile of the low-stage kernel, 2^low_log values
 // per workgroup (11 <= low_log <= min(k, 15) for a transform of k >= 11 stages; 0 = the largest), the
 // stages above it run in strided passes. FFT_LOW_LOOP may be set on top of 15; foreground transforms loop
@@ -36,7 +36,7 @@ struct ColSet {
   int64_t step;
 };
 void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
-                const FftTree& tree, hipStream_t stream, bool background = false, uint32_t low_log = 0);
+                const FftTree& tree, int cus, hipStream_t stream, bool background = false, uint32_t low_log = 0);
 
 // merkle.hip
 void launch_merkle_layer(uint32_t log_size, const uint32_t* prev, const uint32_t* const* cols, uint32_t n_cols,

@@ -252,7 +252,7 @@ void evaluate_into(Ctx& ctx, const std::vector<const uint32_t*>& coeffs, const s
     }
     KScope ks(ctx, K_EVALUATE, (double)idx.size() * (4.0 * (1u << lg) + 4.0 * (1u << target_log)), st);
     ks.units(fft_butterflies(idx.size(), target_log, lg));
-    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, target_log, ctx.fft_tree(false), st, on_side, low);
+    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, target_log, ctx.fft_tree(false), ctx.cu_count, st, on_side, low);
   }
 }
 
@@ -398,7 +398,7 @@ void interpolate_columns(Ctx& ctx, const std::vector<const uint32_t*>& evals, co
     const uint32_t low = ctx.fft_low_log(true, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true));
     KScope ks(ctx, K_INTERPOLATE, (double)idx.size() * 8.0 * (1u << lg));
     ks.units(fft_butterflies(idx.size(), lg, lg));
-    launch_fft(true, d_src, d_dst, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true), ctx.stream, false, low);
+    launch_fft(true, d_src, d_dst, (uint32_t)idx.size(), lg, lg, ctx.fft_tree(true), ctx.cu_count, ctx.stream, false, low);
   }
 }
 
@@ -426,7 +426,7 @@ void evaluate_polynomials(Ctx& ctx, DevTree& t, uint32_t log_blowup) {
     const uint32_t low = ctx.fft_low_log(false, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false));
     KScope ks(ctx, K_EVALUATE, (double)idx.size() * (4.0 * (1u << lg) + 4.0 * (1u << K)));
     ks.units(fft_butterflies(idx.size(), K, lg));
-    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false), ctx.stream, false, low);
+    launch_fft(false, d_src, d_dst, (uint32_t)idx.size(), lg, K, ctx.fft_tree(false), ctx.cu_count, ctx.stream, false, low);
   }
 }
 
