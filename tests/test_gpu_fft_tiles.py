@@ -2,6 +2,8 @@
 loop could go wrong: columns of zeros, of P - 1 and of both in turn (the largest magnitudes that sums and
 differences reach), at every tile size, with a single tile, with more tiles than the device holds
 workgroups (each loops over several), and on columns 4 bytes off 16-byte alignment."""
+import glob
+
 import numpy as np
 import pytest
 
@@ -46,24 +48,46 @@ def test_extreme_values(hb, low, extra):
         assert np.array_equal(w.to_cpu(), O.evaluate(c, log_n + 1))
 
 
-@pytest.mark.parametrize("low,n_cols", [(11, 141), (13, 37), (15, 9)])
-def test_more_tiles_than_workgroups(hb, low, n_cols):
-    """About 4500 tiles of 2^11, 1180 of 2^13 and 290 of 2^15 on unaligned columns."""
-    log_n = 16 if low < 15 else 20
-    print("fft loop", low, log_n, n_cols, flush=True)
+def compute_units():
+    """Of the largest GPU that the kernel driver lists."""
+    best = 0
+    for f in glob.glob("/sys/class/kfd/kfd/topology/nodes/*/properties"):
+        v = dict(line.split() for line in open(f) if len(line.split()) == 2)
+        best = max(best, int(v.get("simd_count", 0)) // max(1, int(v.get("simd_per_cu", 4))))
+    return best or 256
+
+
+@pytest.mark.parametrize("low", [11, 12, 13, 14, 15])
+@pytest.mark.parametrize("above", [0, 2])
+def test_more_tiles_than_workgroups(hb, low, above):
+    """Foreground launches have at most as many workgroups as the device holds at once: here each runs two
+    or three tiles, an uneven number to an XCD; tiles that are whole columns, and four to a column; unaligned
+    columns; forward onto the same domain and, where a tile is a column, onto the twice larger one (two tiles
+    that read the same coefficients)."""
+    resident = (compute_units() // 8 * 8) << (15 - low)
+    n_cols = (resident * 9 // 4 >> above) | 1
+    tiles, log_n = n_cols << above, low + above
+    assert 2 * resident < tiles < 3 * resident and tiles % 8
+    print("fft loop", low, log_n, n_cols, resident, flush=True)
     n = 1 << log_n
-    rng = np.random.default_rng(n_cols)
-    data = rng.integers(0, P, 1 + n_cols * n, dtype=np.uint32)
-    src = hb.from_cpu(data)
-    mid, dst = hb.column(1 + n_cols * n), hb.column(1 + n_cols * n)
-    at = [[c.ptr + 4 * (1 + i * n) for i in range(n_cols)] for c in (src, mid, dst)]
+    data = np.random.default_rng(n_cols).integers(0, P, 1 + n_cols * n, dtype=np.uint32)
+    blow = 1 if above == 0 else 0
+    src, mid, dst = hb.from_cpu(data), hb.column(1 + n_cols * n), hb.column(1 + (n_cols * n << blow))
+    at = lambda c, b=0: [c.ptr + 4 * (1 + (i * n << b)) for i in range(n_cols)]
     hb.set_fft_low_log(low)
     try:
-        hb.interpolate_columns(at[0], log_n, out=at[1])
-        hb.evaluate_polynomials(at[1], log_n, 0, out=at[2])
+        hb.interpolate_columns(at(src), log_n, out=at(mid))
+        hb.evaluate_polynomials(at(mid), log_n, 0, out=at(dst))
+        again = dst.to_cpu()[1:1 + n_cols * n]
+        if blow:
+            hb.evaluate_polynomials(at(mid), log_n, 1, out=at(dst, 1))
     finally:
         hb.set_fft_low_log(0)
-    assert np.array_equal(dst.to_cpu()[1:], data[1:])
-    coeffs = mid.to_cpu()[1:]
-    for i in (0, n_cols // 2, n_cols - 1):
-        assert np.array_equal(coeffs[i * n:(i + 1) * n], O.interpolate(data[1 + i * n:1 + (i + 1) * n]))
+    assert np.array_equal(again, data[1:])
+    coeffs, wide = mid.to_cpu()[1:], dst.to_cpu()[1:]
+    # columns at the ends of the XCDs' ranges
+    for i in sorted({min(n_cols - 1, (n_cols * x >> 3) + d) for x in range(9) for d in (0, 1)} | {n_cols - 2}):
+        c = O.interpolate(data[1 + i * n:1 + (i + 1) * n])
+        assert np.array_equal(coeffs[i * n:(i + 1) * n], c), i
+        if blow:
+            assert np.array_equal(wide[2 * i * n:2 * (i + 1) * n], O.evaluate(c, log_n + 1)), i
