@@ -426,9 +426,8 @@ int stwo_hip_graph_free(stwo_hip_ctx* ctx, stwo_hip_graph* graph);
  * (STWO_HIP_KERNEL_CACHE, else ~/.cache/stwo_hip: fft_plans_<arch>_<CUs>_f64.txt). Results never depend
  * on S. stwo_hip_fft_low_log returns the plan of a shape (tuning it if needed; 0 when the
  * transform has fewer than 11 stages); stwo_hip_set_fft_low_log fixes S for every later transform
- * of the context (clamped to each shape's range; 0 restores planning). A plan may carry the flag
- * 0x100 (S = 15, forward transforms that fill the device); the low-stage kernel runs the same with
- * and without it. */
+ * of the context (clamped to each shape's range; 0 restores planning). The flag 0x100 on S = 15 is
+ * accepted, and reported for forward transforms of 15 stages that fill the device; it changes nothing. */
 int stwo_hip_fft_low_log(stwo_hip_ctx* ctx, int inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
                          uint32_t* low_log);
 int stwo_hip_set_fft_low_log(stwo_hip_ctx* ctx, uint32_t low_log);

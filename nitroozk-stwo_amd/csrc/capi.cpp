@@ -24,6 +24,7 @@ struct stwo_hip_ctx {
   Ctx* ctx = nullptr;
   std::string err;
   std::set<stwo_hip_twiddles*> trees;  // freed with the context if the caller has not
+  bool low_loop = false;               // PLAN_LOOP was given with the fixed tile
 };
 struct stwo_proof {
   ProveResult r;
@@ -1443,12 +1444,16 @@ int stwo_hip_measure_permutation_rate(stwo_hip_ctx* h, double* permutations_per_
   });
 }
 
+// On top of a tile of 2^15 this flag once chose a looping kernel for the low stages. Every foreground
+// transform loops now; the flag is accepted and reported where it was, and reaches no plan.
+constexpr uint32_t PLAN_LOOP = 0x100;
 int stwo_hip_set_fft_low_log(stwo_hip_ctx* h, uint32_t low_log) {
   return guarded(h, [&](Ctx& c) {
-    const uint32_t lg = low_log & ~FFT_LOW_LOOP;
-    if (low_log != 0 && (lg < 11 || lg > 15 || ((low_log & FFT_LOW_LOOP) && lg != 15) || (low_log & ~(FFT_LOW_LOOP | 0xFFu))))
+    const uint32_t lg = low_log & ~PLAN_LOOP;
+    if (low_log != 0 && (lg < 11 || lg > 15 || ((low_log & PLAN_LOOP) && lg != 15)))
       throw HipError(1, "low_log must be 0, 11..15, or 15 with the loop flag 0x100");
-    c.fft_low_override = low_log;
+    c.fft_low_override = lg;
+    h->low_loop = (low_log & PLAN_LOOP) != 0;
   });
 }
 int stwo_hip_fft_low_log(stwo_hip_ctx* h, int inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
@@ -1461,6 +1466,8 @@ int stwo_hip_fft_low_log(stwo_hip_ctx* h, int inverse, uint32_t n_cols, uint32_t
     c.ensure_twiddles(log_n);
     *low_log = inverse ? c.fft_low_log(true, n_cols, log_in, log_n, c.fft_tree(true))
                        : c.fft_low_log(false, n_cols, log_in, log_n, c.fft_tree(false));
+    if (*low_log == 15 && (c.fft_low_override ? h->low_loop : !inverse && log_in == 15 && c.fft_fills(n_cols, log_n - 15)))
+      *low_log |= PLAN_LOOP;
     c.sync();
   });
 }

@@ -607,11 +607,8 @@ void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t 
   if (k >= 11) {
     // stages [0, S) in one pass of 2^S-element blocks; stages [S, k) in strided passes
     const uint32_t smax = k < 15 ? k : 15;
-    const bool loop = (low_log & FFT_LOW_LOOP) != 0;
-    low_log &= ~FFT_LOW_LOOP;
     if (low_log != 0 && (low_log < 11 || low_log > smax)) throw std::invalid_argument("launch_fft: low_log out of range");
     const uint32_t S = low_log ? low_log : smax;
-    if (loop && S != 15) throw std::invalid_argument("launch_fft: FFT_LOW_LOOP needs low_log 15");
     // the stages above the low tile: register passes of at most PASS_REG_MAX stages, as even as
     // the count allows (8 stages: 4 + 4, not 6 + 2)
     std::vector<FftPass> high;

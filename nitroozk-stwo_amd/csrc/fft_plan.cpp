@@ -2,7 +2,7 @@
 //
 // launch_fft runs the stages [0, S) of a transform of k stages in one kernel whose workgroup owns
 // 2^S consecutive values of a column (11 <= S <= min(k, 15), 2^S words of LDS) and the stages
-// [S, k) in strided passes of at most 8 stages. The largest tile reads and writes the data once,
+// [S, k) in register passes of at most 6 stages (PASS_REG_MAX). The largest tile reads and writes the data once,
 // but one workgroup of 2^15 values runs for tens of microseconds, so a transform of few columns
 // (the composition's 4 or 8, the interaction's 32, or 100 columns of 2^16) occupies fewer
 // workgroups than the device has CUs, or ends in a partly filled wave of workgroups. A smaller
@@ -10,12 +10,10 @@
 //
 // The autotuner times every candidate S once per (device, direction, foreground or background,
 // columns, sizes) on scratch columns and keeps the fastest; transforms of at most 15 stages whose
-// largest-tile grid fills the device four times over take S = k without timing (with the flag
-// FFT_LOW_LOOP when forward and S = 15, as plans of that shape always had; launch_fft does the same with
-// and without it), larger ones are timed on a subset of their columns. Choices persist across processes
-// in the cache directory as fft_plans_<arch>_<CUs>_f64.txt (the name changes with the kernels that were
-// timed), one "direction n_cols log_in log_n plan" line per shape (direction: 1 for inverse, plus 2 for
-// a background transform; plan: S, plus 256 for the flag).
+// largest-tile grid fills the device four times over take S = k without timing, larger ones are timed on
+// a subset of their columns. Choices persist across processes in the cache directory as
+// fft_plans_<arch>_<CUs>_f64.txt (the name changes with the kernels that were timed), one "direction
+// n_cols log_in log_n S" line per shape (direction: 1 for inverse, plus 2 for a background transform).
 // STWO_HIP_FFT_TUNE=0 turns the timing off (a fixed rule picks S instead).
 #include <fcntl.h>
 #include <sys/stat.h>
@@ -69,9 +67,8 @@ void load_plans(int device, int cus) {
   if (!fp) return;
   unsigned dir, n, li, ln, s;
   while (std::fscanf(fp, "%u %u %u %u %u", &dir, &n, &li, &ln, &s) == 5) {
-    const uint32_t k = (dir & 1) ? ln : li, tile = s & ~FFT_LOW_LOOP, loop = s & FFT_LOW_LOOP;
-    if (dir < 4 && k >= 11 && tile >= 11 && tile <= std::min<uint32_t>(k, 15) && li <= ln && ln <= 31 &&
-        (s & ~(FFT_LOW_LOOP | 0xFFu)) == 0 && (!loop || (tile == 15 && dir < 2)))
+    const uint32_t k = (dir & 1) ? ln : li;
+    if (dir < 4 && k >= 11 && s >= 11 && s <= std::min<uint32_t>(k, 15) && li <= ln && ln <= 31)
       g_plans[PlanKey{device, dir, n, li, ln}] = s;
   }
   std::fclose(fp);
@@ -97,23 +94,23 @@ bool tuning_enabled() {
 
 }  // namespace
 
+bool Ctx::fft_fills(uint32_t n_cols, uint32_t log_tiles) const {
+  return ((uint64_t)n_cols << log_tiles) >= 4 * (uint64_t)(cu_count > 0 ? cu_count : 1);
+}
+
 uint32_t Ctx::fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree,
                           bool background) {
   const uint32_t k = inverse ? log_n : log_in;
   if (k < 11 || n_cols == 0) return 0;
   const uint32_t smax = k < 15 ? k : 15;
-  if (fft_low_override) {
-    const uint32_t s = std::min(std::max(fft_low_override & ~FFT_LOW_LOOP, 11u), smax);
-    const bool loop = (fft_low_override & FFT_LOW_LOOP) && s == 15 && !background;
-    return s | (loop ? FFT_LOW_LOOP : 0u);
-  }
+  if (fft_low_override) return std::min(std::max(fft_low_override, 11u), smax);
   const uint64_t cus = (uint64_t)(cu_count > 0 ? cu_count : 1);
   if (smax == 11) return smax;
-  const bool fills = ((uint64_t)n_cols << (log_n - smax)) >= 4 * cus;
+  const bool fills = fft_fills(n_cols, log_n - smax);
   // transforms of at most 15 stages that fill the device four times over: one pass of the largest
   // tile (1264 columns of 2^15 onto 2^16: 187 us against 252 to 309 with smaller tiles and a strided pass;
   // the inverse 117 against 142 to 153)
-  if (fills && k <= 15) return smax | (!inverse && !background && smax == 15 ? FFT_LOW_LOOP : 0u);
+  if (fills && k <= 15) return smax;
   const PlanKey key{device, (inverse ? 1u : 0u) + (background ? 2u : 0u), n_cols, log_in, log_n};
   {
     std::lock_guard<std::mutex> lk(g_mu);

@@ -22,12 +22,6 @@ struct FftTree {
   uint32_t len;
 };
 inline size_t fft_tree_doubles(size_t len) { return len < 16 ? 1 : len / 16; }
-// cus: the device's compute units. background: the transform runs beside critical-path kernels on another stream and leaves them the
-// issue priority, and CUs as its tiles end. low_log: the tile of the low-stage kernel, 2^low_log values
-// per workgroup (11 <= low_log <= min(k, 15) for a transform of k >= 11 stages; 0 = the largest), the
-// stages above it run in strided passes. FFT_LOW_LOOP may be set on top of 15; foreground transforms loop
-// over their tiles with any low_log, so it changes nothing.
-constexpr uint32_t FFT_LOW_LOOP = 0x100;
 // The columns of a transform: a device table of addresses, or (null table) column c at base + c step
 // words, which needs no table at all.
 struct ColSet {
@@ -35,6 +29,10 @@ struct ColSet {
   const uint32_t* base;
   int64_t step;
 };
+// cus: the device's compute units. background: the transform runs beside critical-path kernels on another
+// stream and leaves them the issue priority, and CUs as its tiles end. low_log: the tile of the low-stage
+// kernel, 2^low_log values per workgroup (11 <= low_log <= min(k, 15) for a transform of k >= 11 stages;
+// 0 = the largest), the stages above it run in strided passes.
 void launch_fft(bool inverse, ColSet src, ColSet dst, uint32_t n_cols, uint32_t log_in, uint32_t log_n,
                 const FftTree& tree, int cus, hipStream_t stream, bool background = false, uint32_t low_log = 0);
 

@@ -186,6 +186,8 @@ struct Ctx {
   // the transform runs beside critical-path kernels on another stream (planned and timed as such).
   uint32_t fft_low_log(bool inverse, uint32_t n_cols, uint32_t log_in, uint32_t log_n, const FftTree& tree,
                        bool background = false);
+  // Whether n_cols columns of 2^log_tiles tiles fill the device four times over.
+  bool fft_fills(uint32_t n_cols, uint32_t log_tiles) const;
   uint32_t fft_low_override = 0;  // a fixed tile for every shape (stwo_hip_set_fft_low_log); 0 = planned
   int cu_count = 0;
   const uint32_t* domain_xy(uint32_t log);

@@ -2,7 +2,8 @@
 stages above it in strided passes) gives the oracle's interpolation and evaluation, including
 evaluation from fewer coefficients than the domain; the planner keeps the largest tile for
 transforms that fill the device, returns a tile in range otherwise, and persists what it timed.
-The looping kernel (plan flag 0x100) gives the same values."""
+The flag 0x100, which once chose a kernel for tiles of 2^15, is still taken and reported, and changes no
+value (that every tile size loops over many tiles is test_gpu_fft_tiles.py's)."""
 import os
 
 import numpy as np
@@ -28,8 +29,7 @@ def hb():
 
 @pytest.mark.parametrize("low", [11, 12, 13, 14, 15, 15 | 0x100])
 def test_every_tile_matches_the_oracle(hb, low):
-    """0x100: the low stages in the looping kernel (workgroups loop over tiles, next tile
-    prefetched), forward and inverse."""
+    """Forward and inverse; 15 with the flag 0x100 is 15."""
     say("fft tile", low)
     rng = np.random.default_rng(900 + low)
     hb.set_fft_low_log(low)
@@ -51,16 +51,15 @@ def test_plans_are_in_range_and_persist(hb, tmp_path):
     old = os.environ.get("STWO_HIP_KERNEL_CACHE")
     os.environ["STWO_HIP_KERNEL_CACHE"] = str(tmp_path)
     try:
-        # 15 stages filling the device many times over: the largest tile without timing, in the
-        # looping kernel when forward
+        # 15 stages filling the device many times over: the largest tile without timing, reported with
+        # the flag when forward
         assert hb.fft_low_log(False, 4096, 15, 16) == 15 | 0x100
         assert hb.fft_low_log(True, 4096, 15, 15) == 15
         # more stages: timed (on a subset of the columns), a tile in range
         s0 = hb.fft_low_log(True, 4096, 16, 16)
         assert 11 <= (s0 & 0xff) <= 15 and (not s0 & 0x100 or s0 & 0xff == 15)
         assert hb.fft_low_log(False, 7, 10, 12) == 0  # 10 stages: strided passes only
-        # few columns: a timed choice in range, the same on the next query (the looping kernel is a
-        # candidate with 2^15-value tiles)
+        # few columns: a timed choice in range, the same on the next query
         s1 = hb.fft_low_log(True, 5, 17, 17)
         s2 = hb.fft_low_log(False, 3, 14, 16)
         say("planned tiles %#x %#x" % (s1, s2))
@@ -79,9 +78,9 @@ def test_plans_are_in_range_and_persist(hb, tmp_path):
             os.environ["STWO_HIP_KERNEL_CACHE"] = old
 
 
-def test_looping_plan_falls_back_for_unaligned_outputs(hb):
-    """The looping kernel writes 16 bytes at a time; output columns 4 bytes off alignment take the
-    plain kernel under the same plan and still get the oracle's values."""
+def test_unaligned_outputs_under_the_flagged_plan(hb):
+    """The last round writes 16 bytes at a time: output columns 4 bytes off that alignment get the oracle's
+    values under the plan 15 | 0x100, and the plan is reported as it was set."""
     rng = np.random.default_rng(31)
     log_n, n = 15, 2
     cols = [rng.integers(0, P, 1 << log_n, dtype=np.uint32) for _ in range(n)]
@@ -90,6 +89,7 @@ def test_looping_plan_falls_back_for_unaligned_outputs(hb):
     out = [big.ptr + 4 * (1 + i * (2 << log_n)) for i in range(n)]
     hb.set_fft_low_log(15 | 0x100)
     try:
+        assert hb.fft_low_log(True, 2, 15, 15) == 15 | 0x100 and hb.fft_low_log(False, 2, 14, 15) == 14
         hb.evaluate_polynomials(coeffs, log_n, 1, out=out)
     finally:
         hb.set_fft_low_log(0)
