@@ -19,17 +19,16 @@ __device__ __forceinline__ uint32_t mul_tw(uint32_t a, uint32_t t2) {
 // The negation of a doubled twiddle, again doubled: 2P - t2 (0 stays 0).
 __device__ __forceinline__ uint32_t neg_tw(uint32_t t2) { return t2 ? 2 * P - t2 : 0u; }
 
-// NEG: the twiddle is the negation of t2, folded into the butterfly's additions.
-template <bool INV, bool NEG = false>
+template <bool INV>
 __device__ __forceinline__ void bfly(uint32_t& v0, uint32_t& v1, uint32_t t2) {
   const uint32_t a = v0, b = v1;
-  if (INV) {  // ibutterfly(v0, v1, t) = (v0 + v1, (v0 - v1) t); with -t: (v1 - v0) t
+  if (INV) {  // ibutterfly(v0, v1, t) = (v0 + v1, (v0 - v1) t)
     v0 = m31_add(a, b);
-    v1 = mul_tw(NEG ? m31_sub(b, a) : m31_sub(a, b), t2);
-  } else {  // butterfly(v0, v1, t) = (v0 + v1 t, v0 - v1 t); with -t the two swap
+    v1 = mul_tw(m31_sub(a, b), t2);
+  } else {  // butterfly(v0, v1, t) = (v0 + v1 t, v0 - v1 t)
     const uint32_t m = mul_tw(b, t2);
-    v0 = NEG ? m31_sub(a, m) : m31_add(a, m);
-    v1 = NEG ? m31_add(a, m) : m31_sub(a, m);
+    v0 = m31_add(a, m);
+    v1 = m31_sub(a, m);
   }
 }
 
@@ -51,6 +50,7 @@ __device__ __forceinline__ double mul_f64(double b, double t, double M) {
   const double r = __builtin_fma(b, t, -Q);
   return __builtin_fma(Q, 0x1p-31, r);
 }
+// NEG: the twiddle is the negation of t, folded into the butterfly's additions.
 template <bool INV, bool NEG = false>
 __device__ __forceinline__ void bfly_f64(double& v0, double& v1, double t, double M) {
   const double a = v0, b = v1;

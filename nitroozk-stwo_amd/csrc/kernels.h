@@ -185,8 +185,6 @@ void launch_barycentric_weights(uint32_t log_size, cpqm31 p, qm31 vn, const cpm3
 void launch_barycentric_eval(uint32_t log_size, const uint32_t* const* evals, uint32_t n_cols, CCols4 weights,
                              qm31* partial, qm31* out, hipStream_t stream);
 
-void launch_gather_words(const uint32_t* const* bases, const uint32_t* base_idx, const uint32_t* offsets, uint32_t n,
-                         uint32_t* out, hipStream_t stream);
 // Column::batch_at_multi: out[r * n_cols + c] = cols[c][rows[r]]. A gather of at most
 // GATHER_ARG_COLS columns and GATHER_ARG_ROWS rows takes both lists as kernel arguments (no
 // transfer before the launch); a larger one reads them from device tables.

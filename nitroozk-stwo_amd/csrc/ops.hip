@@ -790,19 +790,6 @@ void launch_oods(const OodsTask* tasks, const uint32_t* task_group, uint32_t n_t
                      max_chunks, out);
 }
 
-__global__ void gather_words_kernel(const uint32_t* const* __restrict__ bases, const uint32_t* __restrict__ base_idx,
-                                    const uint32_t* __restrict__ offsets, uint32_t n, uint32_t* __restrict__ out) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = bases[base_idx[i]][offsets[i]];
-}
-
-void launch_gather_words(const uint32_t* const* bases, const uint32_t* base_idx, const uint32_t* offsets, uint32_t n,
-                         uint32_t* out, hipStream_t stream) {
-  if (!n) return;
-  hipLaunchKernelGGL(gather_words_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, bases, base_idx, offsets, n,
-                     out);
-}
-
 // One workgroup. out and flag are coherent host memory: once every lane's stores are visible to the
 // host, the flag takes the call's number, on which the host waits instead of on the stream (the
 // end-of-kernel signal and the runtime's wait for it took longer than the gather: 15.0 us a call
