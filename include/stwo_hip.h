@@ -444,9 +444,10 @@ int stwo_hip_set_kernel_timing(stwo_hip_ctx* ctx, int enable);
  * peak against which VALU-bound kernels (Blake2s hashing, M31 butterflies) are reported. */
 int stwo_hip_measure_int32_issue(stwo_hip_ctx* ctx, double* lane_instr_per_s);
 /* No reference counterpart. The device's forward (inverse != 0: inverse) circle-FFT butterflies per
- * second with the transform kernels' own butterfly code on register-resident values and twiddles:
- * the arithmetic ceiling of the interpolate / evaluate kernels, against which their butterflies per
- * second (stwo_hip_kernel_units over the class's event time) are reported. */
+ * second with the low-stage kernel's own code on register-resident values and twiddles (the
+ * butterflies, and the packing of every value after 5 stages): the arithmetic ceiling of the
+ * interpolate / evaluate kernels, against which their butterflies per second (stwo_hip_kernel_units
+ * over the class's event time) are reported. */
 int stwo_hip_measure_butterfly_rate(stwo_hip_ctx* ctx, int inverse, double* butterflies_per_s);
 /* No reference counterpart. Starknet Poseidon permutations (poseidon_permute_comp) per second on
  * register-resident states with the library's own permutation code: the arithmetic ceiling of

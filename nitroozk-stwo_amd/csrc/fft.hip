@@ -523,7 +523,9 @@ __global__ void __launch_bounds__(LOW_T<S>, 4) fft_low_kernel(ColSet src, ColSet
 
 // Foreground transforms run as many workgroups as the device holds at once, each looping over tiles;
 // a background one has a workgroup per tile, so that the kernels beside it get CUs as its tiles end (a
-// grid that holds every CU until the transform is done doubled the time of the trace's Merkle tree).
+// grid that holds every CU until the transform is done doubled the time of the trace's Merkle tree). Four
+// contexts proving at once do not tell the two forms apart (694-718 proofs/s and p99 7.7-8.2 ms with the
+// resident grid, 692-718 and 8.1-8.6 with a workgroup per tile); a lone one is 1-2 % faster with it.
 template <bool INV, int S>
 static void launch_low_tile(uint32_t n_cols, ColSet src, ColSet dst, uint32_t log_n,
                             uint32_t in_mask, const FftTree& tree, uint32_t rot, uint32_t prio, int cus,
